@@ -120,6 +120,38 @@ inline RowPlan plan_rows(int64_t dim, int elem_bytes, bool aligned, int prefer_n
   return p;
 }
 
+// Workgroups go to the XCDs round robin by block index: block b of n takes the work item that
+// gives each XCD runs of 2^run_log2 consecutive items (a run's blocks are 8 apart); the last
+// n % (8 << run_log2) blocks keep their own index.  A permutation of 0..n-1.
+constexpr int kXcdsLog2 = 3;
+VG_HOST_DEVICE inline uint32_t xcd_item(uint32_t b, uint32_t n, int run_log2) {
+  const int span_log2 = kXcdsLog2 + run_log2;
+  const uint32_t span = b >> span_log2;
+  if (span >= n >> span_log2) return b;
+  const uint32_t r = b & ((1u << span_log2) - 1);
+  return (span << span_log2) + ((r & ((1u << kXcdsLog2) - 1)) << run_log2) + (r >> kXcdsLog2);
+}
+
+// log2 of the workgroups of consecutive rows that one XCD takes in the one-shot forwards (the
+// kernels' xcd_item): about 256 KiB of each stream, 64 workgroups at most.  Consecutive blocks go
+// to different XCDs, so rows by block index spread every 64 KiB of a stream over all eight; runs
+// keep an XCD's requests on neighbouring pages and let the lines that two ragged rows share meet
+// in one L2.  The forward is bound by HBM; measured (bf16, alternating processes, best of 3 to 6;
+// rows by block index / runs of 8, 16, 32 and 64 workgroups, us): 16384 x 4096 86.1 / 86.0, 86.8,
+// 84.1, 89.5; 16384 x 8192 172.1 / 170.3, 169.5, 168.7, 168.8; 8192 x 16384 177.1 / 173.4, 171.8,
+// 173.4, 179.9; 32768 x 2048 86.7 / 88.8, 86.6, 88.4, 84.3; 32768 x 768 35.0 / 34.1, 34.0, 33.6,
+// 33.6; 16384 x 4095 (generic kernel) 100.6 / 97.8, 97.3, 95.8, 94.8; fp32 8192 x 4096 87.5 /
+// 87.9, 86.6, 85.6, 84.7.  Without a residual 16384 x 4096 ran 43.7 against 44.3, quantised to
+// fp8 75.5 against 75.8.  256 KiB is the best or within 2% of it in each.
+constexpr int64_t kXcdRunBytes = 256 << 10;
+constexpr int kXcdRunMaxLog2 = 6;
+inline int xcd_run_log2(int64_t row_bytes, int groups) {
+  const int64_t wg = row_bytes * groups > 0 ? row_bytes * groups : 1;
+  int n = 0;
+  while (n < kXcdRunMaxLog2 && (wg << (n + 1)) * 3 <= kXcdRunBytes * 4) ++n;
+  return n;
+}
+
 // Where the register-resident forward stores h: after the row reduction, beside y, when a row
 // takes at most kLateHMaxTpr threads; before it otherwise.  Measured on MI355X (bf16, A/B in
 // one process, batched launches over rotating buffer sets, 6 rounds): after is faster at dim

@@ -58,6 +58,7 @@ using vg_plan::kMaxWavesPerRow;
 using vg_plan::kWave;
 using vg_plan::max_block_for_nv;
 using vg_plan::RowPlan;
+using vg_plan::xcd_item;
 
 // The weight values of one activation chunk (kVec(DT) columns), kept packed in registers: one
 // 16-byte vector when the weight has the activation dtype, kVec/4 vectors when it is fp32.
@@ -237,6 +238,7 @@ struct FwdArgs {
   float eps;
   float ms_floor;   // > 0: floor on mean(h^2) before eps (the reference module's clamp)
   int64_t rope_seq;       // kOutRopeI: positions per outer index (row position = row % rope_seq)
+  int32_t run_log2;       // log2 of the workgroups of consecutive rows one XCD takes (xcd_item)
   int32_t rope_half;      // kOutRopeI: dim / 2
   float rope_c_hi, rope_c_lo;  // kOutRopeI: log2(base) / half as an unevaluated float sum
 };
@@ -349,7 +351,7 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
   const int grp = threadIdx.x / tpr;
   const int lt = threadIdx.x - grp * tpr;
   const int groups = blockDim.x / tpr;
-  const int64_t row = (int64_t)blockIdx.x * groups + grp;
+  const int64_t row = (int64_t)xcd_item(blockIdx.x, gridDim.x, a.run_log2) * groups + grp;
   const bool row_ok = row < a.rows;
   const int nchunk = a.dim / V;
   const bool has_res = a.res != nullptr;
@@ -941,7 +943,7 @@ __global__ __launch_bounds__(kGenericBlock) void fwd_generic_kernel(const FwdArg
   using C = Codec<DT>;
   using CW = Codec<WDT>;
   __shared__ float red[kGenericBlock / kWave];
-  const int64_t row = blockIdx.x;
+  const int64_t row = xcd_item(blockIdx.x, gridDim.x, a.run_log2);
   const bool has_res = a.res != nullptr;
   const bool has_w = a.w != nullptr;
   const bool write_h = has_res && a.h != nullptr;
@@ -2943,6 +2945,7 @@ int32_t run_fwd(const char* what, int out, const void* x, const void* residual,
   a.eps = eps;
   a.ms_floor = ms_floor;
   a.rope_seq = rope_seq > 0 ? rope_seq : 1;
+  a.run_log2 = vg_plan::xcd_run_log2(dim * eb, p.groups);
   a.rope_half = (int32_t)(dim / 2);
   const double c = (rope_theta > 0.0f && dim >= 2) ? log2((double)rope_theta) / (double)(dim / 2)
                                                    : 0.0;
