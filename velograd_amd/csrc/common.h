@@ -40,6 +40,8 @@ template <>
 struct Codec<VELOGRAD_DTYPE_F32> {
   static constexpr int kBytes = 4;
   static constexpr int kVec = 4;
+  typedef float Raw;  // one stored element
+  __device__ static inline float decode1(Raw v) { return v; }
   __device__ static inline void unpack(const u32x4 v, float* f) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -67,6 +69,10 @@ template <>
 struct Codec<VELOGRAD_DTYPE_BF16> {
   static constexpr int kBytes = 2;
   static constexpr int kVec = 8;
+  typedef uint16_t Raw;
+  __device__ static inline float decode1(Raw v) {
+    return __builtin_bit_cast(float, (uint32_t)v << 16);
+  }
   __device__ static inline void unpack(const u32x4 v, float* f) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -96,6 +102,8 @@ template <>
 struct Codec<VELOGRAD_DTYPE_F16> {
   static constexpr int kBytes = 2;
   static constexpr int kVec = 8;
+  typedef _Float16 Raw;
+  __device__ static inline float decode1(Raw v) { return (float)v; }
   __device__ static inline void unpack(const u32x4 v, float* f) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -187,6 +195,51 @@ __device__ inline void store8_stream(void* base, int64_t elem, const u32x2 v) {
   u32x2* p = reinterpret_cast<u32x2*>(static_cast<char*>(base) + elem * Codec<DT>::kBytes);
 #if VG_STREAM_NT_STORE
   __builtin_nontemporal_store(v, p);
+#else
+  *p = v;
+#endif
+}
+
+// The same 16 bytes starting at any element: gfx950 takes global accesses of any width at any
+// alignment, so one instruction still moves a chunk.  16-byte lanes that straddle lines cost
+// little: rows that start on 4-byte boundaries stream at 5.9-6.4 TB/s, on odd 2-byte ones at
+// 5.2-5.5, against 6.3-6.6 for aligned rows (copy, 2R1W and 2R2W probes at 16384 x 4094 / 4095 /
+// 4096 bf16); shifting dword-aligned loads into place, or stores through the neighbour lane,
+// ran 1-6% slower than this.
+typedef u32x4 u32x4_at2 __attribute__((aligned(2)));
+typedef u32x4 u32x4_at4 __attribute__((aligned(4)));
+template <int BYTES>
+struct AnyAlign {
+  typedef u32x4_at2 chunk;
+};
+template <>
+struct AnyAlign<4> {
+  typedef u32x4_at4 chunk;
+};
+
+template <int DT>
+__device__ inline u32x4 load16_any(const void* base, int64_t elem) {
+  return *reinterpret_cast<const typename AnyAlign<Codec<DT>::kBytes>::chunk*>(static_cast<const char*>(base) +
+                                                                elem * Codec<DT>::kBytes);
+}
+
+template <int DT>
+__device__ inline u32x4 load16_any_stream(const void* base, int64_t elem) {
+  const auto* p = reinterpret_cast<const typename AnyAlign<Codec<DT>::kBytes>::chunk*>(
+      static_cast<const char*>(base) + elem * Codec<DT>::kBytes);
+#if VG_STREAM_NT_LOAD
+  return __builtin_nontemporal_load(p);
+#else
+  return *p;
+#endif
+}
+
+template <int DT>
+__device__ inline void store16_any_stream(void* base, int64_t elem, const u32x4 v) {
+  auto* p = reinterpret_cast<typename AnyAlign<Codec<DT>::kBytes>::chunk*>(static_cast<char*>(base) +
+                                                            elem * Codec<DT>::kBytes);
+#if VG_STREAM_NT_STORE
+  __builtin_nontemporal_store((typename AnyAlign<Codec<DT>::kBytes>::chunk)v, p);
 #else
   *p = v;
 #endif

@@ -120,6 +120,33 @@ inline RowPlan plan_rows(int64_t dim, int elem_bytes, bool aligned, int prefer_n
   return p;
 }
 
+// Rows that the chunked layout does not fit (lengths that are no whole number of 16-byte chunks,
+// streams that start anywhere): fwd_vec_kernel's any-alignment form takes them from one chunk up,
+// laid out over the dim / V whole chunks a row can hold.  Two chunks a thread where a row has
+// enough for that without a residual or with a quantised output (the orders above), else up to
+// kAnyTwoChunks chunks; longer rows one chunk a thread up to the workgroup bound.  Measured with a
+// residual (bf16, 16384 rows; one chunk and h stored early / two chunks and h stored late, us):
+// 1001 26.8 / 25.3, 1535 40.0 / 38.7, 2047 51.6 / 50.0, 3002 71.9 / 70.3, but 4095 95.6 / 98.4 and
+// fp32 8192 x 4099 90.0 / 93.2.
+constexpr int kAnyTwoChunks = 384;
+inline RowPlan plan_any_rows(int64_t dim, int elem_bytes, bool two_first) {
+  RowPlan p{false, 0, kGenericBlock, 1, kGenericBlock};
+  if (elem_bytes != 2 && elem_bytes != 4) return p;
+  const int V = 16 / elem_bytes;
+  if (dim < V) return p;
+  const int64_t chunks = dim / V;
+  const bool two = chunks > kWave && (two_first || chunks <= kAnyTwoChunks);
+  const int nv = two || chunks > max_block_for_nv(1) ? 2 : 1;
+  const int64_t tpr = (chunks + (int64_t)kWave * nv - 1) / ((int64_t)kWave * nv) * kWave;
+  if (tpr > max_block_for_nv(nv)) return p;
+  p.vec = true;
+  p.nv = nv;
+  p.tpr = (int)tpr;
+  p.groups = p.tpr >= 256 ? 1 : 256 / p.tpr;
+  p.block = p.tpr * p.groups;
+  return p;
+}
+
 // Workgroups go to the XCDs round robin by block index: block b of n takes the work item that
 // gives each XCD runs of 2^run_log2 consecutive items (a run's blocks are 8 apart); the last
 // n % (8 << run_log2) blocks keep their own index.  A permutation of 0..n-1.

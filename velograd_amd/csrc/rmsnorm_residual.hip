@@ -79,6 +79,12 @@ struct WeightChunk {
 #pragma unroll
     for (int i = 0; i < kParts; ++i) q[i] = load16<WDT>(w, col0 + i * Codec<WDT>::kVec);
   }
+  // the same from any element of a weight that starts anywhere
+  __device__ inline void load_any(const void* w, int64_t col0) {
+#pragma unroll
+    for (int i = 0; i < kParts; ++i)
+      q[i] = load16_any<WDT>(w, col0 + i * Codec<WDT>::kVec);
+  }
   __device__ inline void unpack(bool has_w, float* f) const {
     if (!has_w) {
 #pragma unroll
@@ -238,8 +244,8 @@ struct FwdArgs {
   float eps;
   float ms_floor;   // > 0: floor on mean(h^2) before eps (the reference module's clamp)
   int64_t rope_seq;       // kOutRopeI: positions per outer index (row position = row % rope_seq)
-  int32_t run_log2;       // log2 of the workgroups of consecutive rows one XCD takes (xcd_item)
   int32_t rope_half;      // kOutRopeI: dim / 2
+  int32_t run_log2;       // log2 of the workgroups of consecutive rows one XCD takes (xcd_item)
   float rope_c_hi, rope_c_lo;  // kOutRopeI: log2(base) / half as an unevaluated float sum
 };
 
@@ -326,6 +332,17 @@ __device__ inline uint32_t lane_group_max(uint32_t v) {
   return v;
 }
 
+// Quantised codes of one chunk at p: aligned to their own size, or (ANY) at any byte.
+template <bool ANY, typename T>
+__device__ inline void store_codes(uint8_t* p, const T v) {
+  if constexpr (ANY) {
+    typedef T AnyT __attribute__((aligned(1)));
+    __builtin_nontemporal_store((AnyT)v, reinterpret_cast<AnyT*>(p));
+  } else {
+    __builtin_nontemporal_store(v, reinterpret_cast<T*>(p));
+  }
+}
+
 // ------------------------------------------------------------------------------------------
 // Forward, register-resident row.
 // ------------------------------------------------------------------------------------------
@@ -334,17 +351,19 @@ __device__ inline uint32_t lane_group_max(uint32_t v) {
 // amax / 448, and y * (1 / scale) is stored as e4m3 codes: 8 bytes per bf16/fp16 chunk, 4 per
 // fp32 chunk.  kOutMxE4M3 / kOutMxE2M1: the 32 elements of an MX block are the chunks of 4
 // (bf16/fp16) or 8 (fp32) consecutive lanes, whose amax is reduced with DPP inside the group.
-// X8: rows of a 2-byte dtype that start on 8-byte boundaries only, dim = n * V + V / 2 (hidden
-// sizes such as 4100; plain outputs only): the row plan covers the n whole chunks, each moved as
-// two 8-byte halves, and the row's last V / 2 elements form an extra half chunk of lane 0 of the
-// row group (every lane of the group loads the same 8 bytes: one request per wave).
-template <int DT, int WDT, int NV, int OUT, bool X8 = false>
+// ANY: rows of any length from one chunk up whose streams start at any element.  The chunks start
+// at the row's first 16-byte boundary of x (the MX blocks at the row's start), and the at most
+// 2 V - 2 elements before and after them go one to a lane.  Streams that sit elsewhere in their
+// 16-byte lines than x are read and written unaligned.
+constexpr int kRowsChunks = 0;    // whole aligned 16-byte chunks
+constexpr int kRowsAnyRes = 1;    // ANY, with a residual
+constexpr int kRowsAnyNoRes = 2;  // ANY, without
+template <int DT, int WDT, int NV, int OUT, int ROWS = kRowsChunks>
 __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const FwdArgs a) {
   using C = Codec<DT>;
   constexpr int V = C::kVec;
-  constexpr int VH = V / 2;
-  static_assert(!X8 || ((OUT == kOutDtype || OUT == kOutDtypeLateH) && C::kBytes == 2),
-                "rows of 8-byte alignment: plain outputs of a 2-byte dtype");
+  constexpr bool ANY = ROWS != kRowsChunks;
+  static_assert(!ANY || OUT != kOutRopeDirect, "the RoPE output takes aligned rows here");
   __shared__ float red[kMaxWavesPerRow];
 
   const int tpr = a.tpr;
@@ -353,28 +372,24 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
   const int groups = blockDim.x / tpr;
   const int64_t row = (int64_t)xcd_item(blockIdx.x, gridDim.x, a.run_log2) * groups + grp;
   const bool row_ok = row < a.rows;
-  const int nchunk = a.dim / V;
-  const bool has_res = a.res != nullptr;
+  constexpr bool MX = OUT == kOutMxE4M3 || OUT == kOutMxE2M1;
+  int head = 0;
+  if constexpr (ANY && !MX) {
+    const int off = (int)row_offset16(a.x, row * a.ld_x, C::kBytes);
+    head = min(((16 - off) & 15) / C::kBytes, a.dim);
+  }
+  const int nchunk = (a.dim - head) / V;
+  // (known at compile time for ANY: a branch on it would put waits between the loads)
+  const bool has_res = ANY ? ROWS == kRowsAnyRes : a.res != nullptr;
   const bool has_w = a.w != nullptr;
-  const int64_t xcol = (int64_t)a.dim - VH;  // X8: the extra half chunk's first column
-  const bool own_x = X8 && lt == 0;
-  // One chunk of a stream: 16 bytes, or two 8-byte halves for X8 rows.
+  auto col_of = [&](int c) -> int { return head + c * V; };
   auto load_chunk = [&](const void* base, int64_t e) -> u32x4 {
-    if constexpr (X8) {
-      const u32x2 lo = load8_stream<DT>(base, e);
-      const u32x2 hi = load8_stream<DT>(base, e + VH);
-      return u32x4{lo.x, lo.y, hi.x, hi.y};
-    } else {
-      return load16_stream<DT>(base, e);
-    }
+    if constexpr (ANY) return load16_any_stream<DT>(base, e);
+    else return load16_stream<DT>(base, e);
   };
   auto store_chunk = [&](void* base, int64_t e, const u32x4 v) {
-    if constexpr (X8) {
-      store8_stream<DT>(base, e, u32x2{v.x, v.y});
-      store8_stream<DT>(base, e + VH, u32x2{v.z, v.w});
-    } else {
-      store16_stream<DT>(base, e, v);
-    }
+    if constexpr (ANY) store16_any_stream<DT>(base, e, v);
+    else store16_stream<DT>(base, e, v);
   };
 
   // Only the packed 16-byte chunks stay live across the row reduction; fp32 h is formed again
@@ -382,54 +397,47 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
   // up to 8 chunks per thread.
   u32x4 xv[NV], rv[NV];
   WeightChunk<DT, WDT> wc[NV];
-#pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const int c = lt + k * tpr;
-    xv[k] = u32x4{0u, 0u, 0u, 0u};
-    rv[k] = u32x4{0u, 0u, 0u, 0u};
-    if (row_ok && c < nchunk) {
-      xv[k] = load_chunk(a.x, row * a.ld_x + (int64_t)c * V);
-      if (has_res) rv[k] = load_chunk(a.res, row * a.ld_res + (int64_t)c * V);
+  // ANY: the lane's element outside the chunks
+  const bool own_s = ANY && row_ok && lt < a.dim - nchunk * V;
+  const int j_s = lt < head ? lt : lt + nchunk * V;
+  typename C::Raw x_raw{}, r_raw{};
+  typename Codec<WDT>::Raw w_raw{};
+  if constexpr (ANY) {
+    // No wait may fall between these loads (16384 x 4095 bf16 100.9 us with one, 94.2 without), so
+    // the raw elements come first and are decoded at the row sum, what is absent is
+    // read from x instead, a lane without a chunk reads the row's last columns and a row past
+    // the end reads the last row.
+    if (own_s) {
+      x_raw = static_cast<const typename C::Raw*>(a.x)[row * a.ld_x + j_s];
+      if (has_res) r_raw = static_cast<const typename C::Raw*>(a.res)[row * a.ld_res + j_s];
+      w_raw = static_cast<const typename Codec<WDT>::Raw*>(has_w ? a.w : a.x)[has_w ? j_s : 0];
     }
-  }
-  u32x2 xx = u32x2{0u, 0u}, rx = u32x2{0u, 0u};
-  float wfx[VH];
-  if constexpr (X8) {
-    if (row_ok) {
-      xx = load8_stream<DT>(a.x, row * a.ld_x + xcol);
-      if (has_res) rx = load8_stream<DT>(a.res, row * a.ld_res + xcol);
+    const int64_t rw = row_ok ? row : a.rows - 1;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int col = min(col_of(lt + k * tpr), a.dim - V);
+      xv[k] = load_chunk(a.x, rw * a.ld_x + col);
+      if (has_res) rv[k] = load_chunk(a.res, rw * a.ld_res + col);
+      if (has_w) wc[k].load_any(a.w, col);
     }
+  } else {
 #pragma unroll
-    for (int i = 0; i < VH; ++i) wfx[i] = 1.0f;
-    if (has_w) {
-      if constexpr (WDT == VELOGRAD_DTYPE_F32) {
-        Codec<VELOGRAD_DTYPE_F32>::unpack(load16<VELOGRAD_DTYPE_F32>(a.w, xcol), wfx);
-      } else {
-        const u32x2 q = *reinterpret_cast<const u32x2*>(static_cast<const char*>(a.w) +
-                                                        xcol * Codec<WDT>::kBytes);
-        float t[V];
-        Codec<WDT>::unpack(u32x4{q.x, q.y, 0u, 0u}, t);
-#pragma unroll
-        for (int i = 0; i < VH; ++i) wfx[i] = t[i];
+    for (int k = 0; k < NV; ++k) {
+      const int c = lt + k * tpr;
+      xv[k] = u32x4{0u, 0u, 0u, 0u};
+      rv[k] = u32x4{0u, 0u, 0u, 0u};
+      if (row_ok && c < nchunk) {
+        xv[k] = load_chunk(a.x, row * a.ld_x + (int64_t)c * V);
+        if (has_res) rv[k] = load_chunk(a.res, row * a.ld_res + (int64_t)c * V);
       }
     }
-  }
 #pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const int c = lt + k * tpr;
-    wc[k].load((has_w && c < nchunk) ? a.w : nullptr, (int64_t)c * V);
+    for (int k = 0; k < NV; ++k) {
+      const int c = lt + k * tpr;
+      wc[k].load((has_w && c < nchunk) ? a.w : nullptr, (int64_t)c * V);
+    }
   }
 
-  // the extra half chunk's h (X8), in the first VH of V slots, the rest 0
-  auto make_hx = [&](float* hf) {
-    C::unpack(u32x4{xx.x, xx.y, 0u, 0u}, hf);
-    if (has_res) {
-      float rf[V];
-      C::unpack(u32x4{rx.x, rx.y, 0u, 0u}, rf);
-#pragma unroll
-      for (int i = 0; i < VH; ++i) hf[i] = hf[i] + rf[i];
-    }
-  };
   auto make_h = [&](int k, float* hf) {
     C::unpack(xv[k], hf);
     if (has_res) {
@@ -447,25 +455,29 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
   for (int k = 0; k < NV; ++k) {
     float hf[V];
     make_h(k, hf);
-#pragma unroll
-    for (int i = 0; i < V; ++i) ss += hf[i] * hf[i];
     const int c = lt + k * tpr;
-    if (!kLateH && write_h && row_ok && c < nchunk)
-      store_chunk(a.h, row * a.ld_h + (int64_t)c * V, C::pack(hf));
-  }
-  if constexpr (X8) {
-    float hf[V];
-    make_hx(hf);
-    float p = 0.0f;
+    if constexpr (ANY) {
+      float p = 0.0f;
 #pragma unroll
-    for (int i = 0; i < VH; ++i) p += hf[i] * hf[i];
-    ss += own_x ? p : 0.0f;
-    if (!kLateH && write_h && row_ok && own_x) {
-      const u32x4 pv = C::pack(hf);
-      store8_stream<DT>(a.h, row * a.ld_h + xcol, u32x2{pv.x, pv.y});
+      for (int i = 0; i < V; ++i) p += hf[i] * hf[i];
+      ss += c < nchunk ? p : 0.0f;
+    } else {
+#pragma unroll
+      for (int i = 0; i < V; ++i) ss += hf[i] * hf[i];
     }
+    if (!kLateH && write_h && row_ok && c < nchunk)
+      store_chunk(a.h, row * a.ld_h + col_of(c), C::pack(hf));
   }
 
+  float h_s = 0.0f, w_s = 1.0f;
+  if constexpr (ANY) {
+    asm volatile("" : "+v"(x_raw), "+v"(r_raw), "+v"(w_raw));  // no decoding before this point
+    h_s = C::decode1(x_raw);
+    if (has_res) h_s = h_s + C::decode1(r_raw);
+    if (has_w) w_s = Codec<WDT>::decode1(w_raw);
+    ss += h_s * h_s;
+    if (write_h && own_s) C::store1(a.h, row * a.ld_h + j_s, h_s);
+  }
   ss = row_sum(ss, tpr, grp, red);
   const float mean_sq = floor_mean_sq(ss / (float)a.dim, a.ms_floor);
   const float r = 1.0f / __builtin_sqrtf(mean_sq + a.eps);
@@ -495,7 +507,7 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
         if (kLateH && write_h) {
           float hf[V];
           make_h(k, hf);
-          store_chunk(a.h, row * a.ld_h + (int64_t)c * V, C::pack(hf));
+          store_chunk(a.h, row * a.ld_h + col_of(c), C::pack(hf));
         }
         float yf[V];
         make_y(k, yf);
@@ -513,27 +525,13 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
             yf[2 * q + 1] = y0 * sn + y1 * cs;                             // functional.py:314
           }
         }
-        store_chunk(a.y, row * a.ld_y + (int64_t)c * V, C::pack(yf));
+        store_chunk(a.y, row * a.ld_y + col_of(c), C::pack(yf));
       }
     }
-    if constexpr (X8) {
-      if (row_ok && own_x) {
-        float hf[V];
-        make_hx(hf);
-        if (kLateH && write_h) {
-          const u32x4 pv = C::pack(hf);
-          store8_stream<DT>(a.h, row * a.ld_h + xcol, u32x2{pv.x, pv.y});
-        }
-        float yf[V];
-#pragma unroll
-        for (int i = 0; i < VH; ++i) yf[i] = (hf[i] * r) * wfx[i];
-#pragma unroll
-        for (int i = VH; i < V; ++i) yf[i] = 0.0f;
-        const u32x4 pv = C::pack(yf);
-        store8_stream<DT>(a.y, row * a.ld_y + xcol, u32x2{pv.x, pv.y});
-      }
+    if constexpr (ANY) {
+      if (own_s) C::store1(a.y, row * a.ld_y + j_s, (h_s * r) * w_s);
     }
-  } else if constexpr (OUT == kOutMxE4M3 || OUT == kOutMxE2M1) {
+  } else if constexpr (MX) {
     constexpr int kEmax = OUT == kOutMxE4M3 ? vg_mx::kEmaxE4M3 : vg_mx::kEmaxE2M1;
     constexpr int kLanes = vg_mx::kBlock / V;  // lanes per MX block
 #pragma unroll
@@ -561,9 +559,9 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
           }
           if constexpr (V == 8) {
             const u32x2 w2 = {words[0], words[1]};
-            __builtin_nontemporal_store(w2, reinterpret_cast<u32x2*>(dst + (int64_t)c * V));
+            store_codes<ANY>(dst + (int64_t)c * V, w2);
           } else {
-            __builtin_nontemporal_store(words[0], reinterpret_cast<uint32_t*>(dst + (int64_t)c * V));
+            store_codes<ANY>(dst + (int64_t)c * V, words[0]);
           }
         } else {
           uint32_t word = 0;
@@ -575,10 +573,9 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
           }
           if (!finite) word = 0;
           if constexpr (V == 8) {
-            __builtin_nontemporal_store(word, reinterpret_cast<uint32_t*>(dst + (int64_t)c * 4));
+            store_codes<ANY>(dst + (int64_t)c * 4, word);
           } else {
-            __builtin_nontemporal_store((uint16_t)word,
-                                        reinterpret_cast<uint16_t*>(dst + (int64_t)c * 2));
+            store_codes<ANY>(dst + (int64_t)c * 2, (uint16_t)word);
           }
         }
         if (lt % kLanes == 0)
@@ -600,6 +597,10 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
           am = umax(am, __builtin_bit_cast(uint32_t, yf[k][i]) & 0x7fffffffu);
       }
     }
+    const float y_s = (h_s * r) * w_s;
+    if constexpr (ANY) {
+      if (own_s) am = umax(am, __builtin_bit_cast(uint32_t, y_s) & 0x7fffffffu);
+    }
     am = row_max_abs_bits(am, tpr, grp, red_max);
     const float scale = __builtin_bit_cast(float, am) / kE4M3Max;
     const float inv = inverse_scale(scale);
@@ -614,14 +615,17 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
           words[j] = e4m3x4(yf[k][4 * j] * inv, yf[k][4 * j + 1] * inv, yf[k][4 * j + 2] * inv,
                             yf[k][4 * j + 3] * inv);
         }
-        uint8_t* dst = static_cast<uint8_t*>(a.y) + row * a.ld_y + (int64_t)c * V;
+        uint8_t* dst = static_cast<uint8_t*>(a.y) + row * a.ld_y + col_of(c);
         if constexpr (V == 8) {
           const u32x2 w2 = {words[0], words[1]};
-          __builtin_nontemporal_store(w2, reinterpret_cast<u32x2*>(dst));
+          store_codes<ANY>(dst, w2);
         } else {
-          __builtin_nontemporal_store(words[0], reinterpret_cast<uint32_t*>(dst));
+          store_codes<ANY>(dst, words[0]);
         }
       }
+    }
+    if constexpr (ANY) {
+      if (own_s) static_cast<uint8_t*>(a.y)[row * a.ld_y + j_s] = (uint8_t)e4m3x1(y_s * inv);
     }
   }
 }
@@ -850,15 +854,13 @@ __global__ __launch_bounds__(max_block_for_nv(1)) void fwd_rope_kernel(const Fwd
 }
 
 // ------------------------------------------------------------------------------------------
-// Forward, rows of any length and alignment up to 4096 elements that the chunked kernels cannot
-// take (odd lengths, streams that start anywhere inside a 16-byte line): one-shot rows as in
-// fwd_vec_kernel, several short rows a workgroup, with bwd_ring_elem_kernel's element-strided
-// lanes (lane lt of a row group holds columns lt, lt + tpr, ..., M of them), so each of a
-// wave's element loads and stores moves one contiguous run of 64 elements.  y in the activation
-// dtype (the plain output) only; short rows (kFwdElemMaxDim), where the generic kernel's one row
-// per workgroup is bound by each row's latency.
+// Forward, short rows of any length and alignment (kFwdElemMaxDim): one-shot rows as in
+// fwd_vec_kernel, several a workgroup, with bwd_ring_elem_kernel's element-strided lanes (lane lt
+// of a row group holds columns lt, lt + tpr, ..., M of them), so each of a wave's element loads
+// and stores moves one contiguous run of 64 elements.  y in the activation dtype (the plain
+// output) only; longer rows move in chunks (fwd_vec_kernel's ANY).
 // ------------------------------------------------------------------------------------------
-constexpr int64_t kFwdElemMaxDim = 1024;  // the host plans it for rows of at most this length
+constexpr int64_t kFwdElemMaxDim = 64;  // the host plans it for rows of at most this length
 
 template <int DT, int WDT, int M>
 __global__ __launch_bounds__(vg_plan::kRingBlock) void fwd_elem_kernel(const FwdArgs a) {
@@ -935,7 +937,9 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void fwd_elem_kernel(const Fwd
 }
 
 // ------------------------------------------------------------------------------------------
-// Forward, any dim / alignment: one row per workgroup, two passes over the row (the second
+// Forward, the rows that the kernels above do not take (longer than their registers hold, shorter
+// than a chunk with a quantised output, the RoPE output on rows that are not whole chunks, streams
+// off their element's alignment): one row per workgroup, two passes over the row (the second
 // re-reads x and residual, normally from L2, and recomputes the identical fp32 h).
 // ------------------------------------------------------------------------------------------
 template <int DT, int WDT, int OUT>
@@ -2520,6 +2524,9 @@ BwdPlan plan_bwd(int64_t rows, int64_t dim, int elem_bytes, bool aligned, bool a
 
 bool ld_ok(int64_t ld, int elem_bytes) { return ((ld * elem_bytes) & 15) == 0; }
 bool ld_ok8(int64_t ld, int elem_bytes) { return ((ld * elem_bytes) & 7) == 0; }
+bool elem_ok_ptr(const void* p, int bytes) {
+  return (reinterpret_cast<uintptr_t>(p) & (uintptr_t)(bytes - 1)) == 0;
+}
 bool aligned8p(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7) == 0; }
 
 // ------------------------------------------------------------------------------------------
@@ -2604,30 +2611,27 @@ void launch_fwd(const FwdArgs& a, const RowPlan& p, hipStream_t st) {
   }
 }
 
-// Rows of 8-byte alignment (fwd_vec_kernel's X8): `p` lays out the dim - V / 2 columns of whole
-// chunks.
-template <int DT, int WDT>
-void launch_fwd_x8(const FwdArgs& a, const RowPlan& p, hipStream_t st) {
-  if constexpr (Codec<DT>::kBytes == 2) {
-    const dim3 grid((uint32_t)((a.rows + p.groups - 1) / p.groups)), block(p.block);
-    const bool late = vg_plan::fwd_late_h(p);
-    switch (p.nv * 2 + (late ? 1 : 0)) {
-#define VG_FWD_X8(N)                                                                          \
-  case 2 * (N):                                                                               \
-    hipLaunchKernelGGL((fwd_vec_kernel<DT, WDT, N, kOutDtype, true>), grid, block, 0, st, a); \
-    break;                                                                                    \
-  case 2 * (N) + 1:                                                                           \
-    hipLaunchKernelGGL((fwd_vec_kernel<DT, WDT, N, kOutDtypeLateH, true>), grid, block, 0, st, \
-                       a);                                                                    \
-    break;
-      VG_FWD_X8(1)
-      VG_FWD_X8(2)
-      VG_FWD_X8(3)
-      VG_FWD_X8(4)
-#undef VG_FWD_X8
-      default: break;
+// Rows of any length and alignment (fwd_vec_kernel's ANY), planned by plan_any_rows.
+template <int DT, int WDT, int OUT, int ROWS>
+void launch_fwd_any_rows(const FwdArgs& a, const RowPlan& p, hipStream_t st) {
+  const dim3 grid((uint32_t)((a.rows + p.groups - 1) / p.groups)), block(p.block);
+  if (p.nv == 1) {
+    hipLaunchKernelGGL((fwd_vec_kernel<DT, WDT, 1, OUT, ROWS>), grid, block, 0, st, a);
+    return;
+  }
+  if constexpr (OUT == kOutDtype && ROWS == kRowsAnyRes) {
+    if (vg_plan::fwd_late_h(p)) {
+      hipLaunchKernelGGL((fwd_vec_kernel<DT, WDT, 2, kOutDtypeLateH, ROWS>), grid, block, 0, st, a);
+      return;
     }
   }
+  hipLaunchKernelGGL((fwd_vec_kernel<DT, WDT, 2, OUT, ROWS>), grid, block, 0, st, a);
+}
+
+template <int DT, int WDT, int OUT>
+void launch_fwd_any(const FwdArgs& a, const RowPlan& p, hipStream_t st) {
+  if (a.res != nullptr) launch_fwd_any_rows<DT, WDT, OUT, kRowsAnyRes>(a, p, st);
+  else launch_fwd_any_rows<DT, WDT, OUT, kRowsAnyNoRes>(a, p, st);
 }
 
 // Rows of element-strided lanes (fwd_elem_kernel): `p` from plan_elem_rows, m elements a lane.
@@ -2894,34 +2898,34 @@ int32_t run_fwd(const char* what, int out, const void* x, const void* residual,
   // (one chunk first) either way.
   RowPlan p = plan_fwd(dim, eb, aligned, residual == nullptr && out != kOutRopeI,
                        out == kOutFp8Row || mx);
-  // Rows of 8n + 4 two-byte elements on 8-byte boundaries (fwd_vec_kernel's X8): the plan of
-  // their whole chunks, the last 4 elements an extra half chunk.
-  const bool aligned8 = aligned8p(x) && ld_ok8(ld_x, eb) && aligned8p(y) && ld_ok8(ld_y, eb) &&
-                        (!residual || (aligned8p(residual) && ld_ok8(ld_res, eb))) &&
-                        (!h || (aligned8p(h) && ld_ok8(ld_h, eb))) &&
-                        (!weight || aligned16(weight));
-  bool x8 = false;
-  if (!p.vec && out == kOutDtype && eb == 2 && dim >= 12 && dim % 8 == 4 && aligned8) {
-    const RowPlan px = plan_fwd(dim - 4, eb, true, residual == nullptr, false);
-    if (px.vec) {
-      p = px;
-      x8 = true;
-    }
-  }
-  // other short rows the chunked kernels cannot take: element-strided lanes, several rows a
-  // workgroup.  Longer rows keep the generic kernel, whose row middles move in 16-byte accesses:
-  // bf16 16384 x 99 10.6 us against 38.6 in the generic kernel, 255 13.3 against 40.2, 1001 46.6
-  // against 49.2, but 2047 85.9 against 60.2, 3001 154.3 against 81.4, 4095 161.5 against 100.4.
+  // rows the chunked layout does not fit, on element boundaries
+  const bool aligned_elem = elem_ok_ptr(x, eb) && (out != kOutDtype || elem_ok_ptr(y, eb)) &&
+                            elem_ok_ptr(residual, eb) && elem_ok_ptr(h, eb) &&
+                            elem_ok_ptr(weight, elem_bytes_of(w_dtype));
+  // The shortest of them go element by element, several rows a workgroup; the others in chunks
+  // from any element (plan_any_rows), longer ones than that fits in the generic kernel.  Measured
+  // on MI355X, 16384 rows with a residual, the kernels before (elements up to 1024, the generic
+  // kernel past them) / chunks, us: bf16 17 7.2 / 8.7, 99 10.0 / 9.8, 255 14.0 / 10.8, 1001 45.4 /
+  // 24.4, 2047 59.2 / 50.6, 4095 99.7 / 94.2, 8192 x 8191 103.2 / 93.3, 8192 x 12001 146.4 / 137.2,
+  // fp32 1001 57.9 / 47.5, 8192 x 4099 105.8 / 90.6; rows of 8n + 4 elements in 8-byte halves 4100
+  // 93.0 / 92.4, 2052 48.4 / 48.7; without a residual 2047 41.3 / 25.8; quantised to fp8 (generic
+  // kernel) 255 30.6 / 11.3, 2047 192 / 44.4, 4095 404 / 86.4.
+  bool any = false;
   int elem_m = 0;
-  if (!p.vec && !x8 && out == kOutDtype && (eb == 2 || eb == 4) && dim <= kFwdElemMaxDim &&
-      tuning().fwd_elem) {
+  if (!p.vec && out == kOutDtype && dim <= kFwdElemMaxDim && tuning().fwd_elem) {
     elem_m = vg_plan::elem_per_lane(dim);
     if (elem_m > 0) p = vg_plan::plan_elem_rows(dim);
+  } else if (!p.vec && out != kOutRopeI && aligned_elem) {
+    const RowPlan pa = vg_plan::plan_any_rows(dim, eb, residual == nullptr || out != kOutDtype);
+    if (pa.vec) {
+      p = pa;
+      any = true;
+    }
   }
   const bool elem_ok = p.tpr % kWave == 0 && p.tpr >= kWave && p.groups >= 1 &&
                        p.block == p.tpr * p.groups && p.block <= vg_plan::kRingBlock &&
                        (int64_t)elem_m * p.tpr >= dim;
-  if (elem_m > 0 ? !elem_ok : !vg_plan::row_plan_valid(p, x8 ? dim - 4 : dim, eb))
+  if (elem_m > 0 ? !elem_ok : !vg_plan::row_plan_valid(p, any ? dim / (16 / eb) * (16 / eb) : dim, eb))
     return fail(VELOGRAD_ERR_INVALID_ARGUMENT, "%s: internal launch plan rejected (dim=%lld)",
                 what, (long long)dim);
 
@@ -2945,21 +2949,29 @@ int32_t run_fwd(const char* what, int out, const void* x, const void* residual,
   a.eps = eps;
   a.ms_floor = ms_floor;
   a.rope_seq = rope_seq > 0 ? rope_seq : 1;
-  a.run_log2 = vg_plan::xcd_run_log2(dim * eb, p.groups);
   a.rope_half = (int32_t)(dim / 2);
+  a.run_log2 = vg_plan::xcd_run_log2(dim * eb, p.groups);
   const double c = (rope_theta > 0.0f && dim >= 2) ? log2((double)rope_theta) / (double)(dim / 2)
                                                    : 0.0;
   a.rope_c_hi = (float)c;
   a.rope_c_lo = (float)(c - (double)a.rope_c_hi);
   hipStream_t st = static_cast<hipStream_t>(hip_stream);
   switch (out) {
-    case kOutFp8Row: VG_DISPATCH_TYPES(dtype, w_dtype, (launch_fwd<kD, kW, kOutFp8Row>(a, p, st))); break;
-    case kOutMxE4M3: VG_DISPATCH_TYPES(dtype, w_dtype, (launch_fwd<kD, kW, kOutMxE4M3>(a, p, st))); break;
-    case kOutMxE2M1: VG_DISPATCH_TYPES(dtype, w_dtype, (launch_fwd<kD, kW, kOutMxE2M1>(a, p, st))); break;
+#define VG_FWD_OUT(O)                                                                  \
+  case O:                                                                              \
+    if (any)                                                                           \
+      VG_DISPATCH_TYPES(dtype, w_dtype, (launch_fwd_any<kD, kW, O>(a, p, st)));        \
+    else                                                                               \
+      VG_DISPATCH_TYPES(dtype, w_dtype, (launch_fwd<kD, kW, O>(a, p, st)));            \
+    break;
+    VG_FWD_OUT(kOutFp8Row)
+    VG_FWD_OUT(kOutMxE4M3)
+    VG_FWD_OUT(kOutMxE2M1)
+#undef VG_FWD_OUT
     case kOutRopeI: VG_DISPATCH_TYPES(dtype, w_dtype, (launch_fwd<kD, kW, kOutRopeI>(a, p, st))); break;
     default:
-      if (x8)
-        VG_DISPATCH_TYPES(dtype, w_dtype, (launch_fwd_x8<kD, kW>(a, p, st)));
+      if (any)
+        VG_DISPATCH_TYPES(dtype, w_dtype, (launch_fwd_any<kD, kW, kOutDtype>(a, p, st)));
       else if (elem_m > 0)
         VG_DISPATCH_TYPES(dtype, w_dtype, (launch_fwd_elem<kD, kW>(a, p, elem_m, st)));
       else
