@@ -540,15 +540,45 @@ inline BwdPlan plan_bwd_rope(int64_t rows, int64_t dim, int elem_bytes, bool ali
                   kBwdOrderRope);
 }
 
-// Rows per walk of the norm + RoPE forward (fwd_rope_kernel: workgroup b walks rows b, b + G, ...
-// with G = ceil(rows / W)).  32-row walks halve the workgroups and the per-walk set-up (the
-// step and first rotations, a few hundred vector instructions a thread); they pay where a row
-// group fills a CU's waves with fewer workgroups (more than 256 threads) and the tensor keeps
-// at least two 32-row walks per CU on 256 CUs.  Measured on MI355X (bf16, module form, A/B in one
-// process, 3 rounds; 16-row against 32-row walks): 16384 x 4096 51.2 / 50.0 us (one sequence
-// 50.3 / 49.8), 16384 x 5120 73.4 / 61.4, 16384 x 7168 98.2 / 89.5, 16384 x 8192 103.8 / 94.1,
-// 16384 x 3072 42.1 / 40.3; against: 32768 x 2048 51.6 / 52.2 (256-thread rows), 8192 x 4096
-// 27.2 / 31.2 (256 workgroups); 64-row walks lost everywhere (99.6 us at 16384 x 4096).
+// Tiles of the norm + RoPE forward (fwd_rope_tile_kernel): row groups of one chunk a thread up to
+// the workgroup bound (the row's last chunk may overlap the one before it), else of two; tiles of
+// four consecutive positions, two with a residual (its loads double the registers: 16384 x 4096
+// bf16 88.2 us against 91.6, 8192 x 16384 195 against 259), halved while they are longer than the
+// sequence or leave fewer than kRopeTileMinWgs workgroups (bf16 dim 4096, tiles of 1 / 2 / 4, us: 64
+// rows 3.5 / 3.9 / 4.5, 512 4.8 / 4.4 / 5.0, 2048 11.7 / 8.8 / 8.1).  `rp.vec` false: a row shorter
+// than a chunk or longer than the registers hold.
+struct RopeTilePlan {
+  RowPlan rp;
+  int tile;     // positions a tile
+  int64_t wgs;  // workgroups, rp.groups tiles each
+};
+constexpr int64_t kRopeTileMinWgs = 256;
+
+inline RopeTilePlan plan_rope_tiles(int64_t rows, int64_t dim, int elem_bytes, int64_t seq,
+                                    bool residual) {
+  RopeTilePlan t{RowPlan{false, 0, kGenericBlock, 1, kGenericBlock}, 1, 0};
+  if ((elem_bytes != 2 && elem_bytes != 4) || rows < 1 || seq < 1) return t;
+  const int V = 16 / elem_bytes;
+  if (dim < V) return t;
+  const int64_t chunks = (dim + V - 1) / V;
+  const int nv = chunks > max_block_for_nv(1) ? 2 : 1;
+  const int64_t tpr = (chunks + (int64_t)kWave * nv - 1) / ((int64_t)kWave * nv) * kWave;
+  if (tpr > max_block_for_nv(nv)) return t;
+  RowPlan& p = t.rp;
+  p.vec = true;
+  p.nv = nv;
+  p.tpr = (int)tpr;
+  p.groups = p.tpr >= 256 ? 1 : 256 / p.tpr;
+  p.block = p.tpr * p.groups;
+  auto wgs = [&](int r) { return (rows / seq * ((seq + r - 1) / r) + p.groups - 1) / p.groups; };
+  t.tile = residual ? 2 : 4;
+  while (t.tile > 1 && (t.tile > seq || wgs(t.tile) < kRopeTileMinWgs)) t.tile /= 2;
+  t.wgs = wgs(t.tile);
+  return t;
+}
+
+// Rows a workgroup walked in the strided norm + RoPE forward that fwd_rope_tile_kernel replaced
+// (no kernel takes it any more; the planner's test still states it).
 constexpr int kNormRopeRows = 16;
 constexpr int kNormRopeLongRows = 32;
 constexpr int64_t kNormRopeLongMinRows = 16384;

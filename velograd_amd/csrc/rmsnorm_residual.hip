@@ -25,8 +25,8 @@
 //                       row buffers (two rows in flight while one reduces) in a branch-free
 //                       steady loop, 512-thread workgroups, one per CU: the backward's default
 //                       where the rows suit it.
-//   fwd_rope_kernel     the forward with the model's interleaved RoPE on y: strided row walks
-//                       with the rotation advanced by a recurrence.
+//   fwd_rope_tile_kernel  the forward with the model's interleaved RoPE on y: short tiles of
+//                       consecutive positions, the rotation advanced by a recurrence in each.
 //   bwd_rope_ring_kernel  its backward (grad_y rotated back, then the norm's backward) in
 //                       bwd_ring_kernel's walk, one or two chunks per thread (rows of up to
 //                       1024 chunks), one workgroup per CU (two of one chunk and under 512
@@ -247,6 +247,8 @@ struct FwdArgs {
   int32_t rope_half;      // kOutRopeI: dim / 2
   int32_t run_log2;       // log2 of the workgroups of consecutive rows one XCD takes (xcd_item)
   float rope_c_hi, rope_c_lo;  // kOutRopeI: log2(base) / half as an unevaluated float sum
+  double rope_log2_step, rope_ratio;  // kOutRopeI: -log2(base) / half and 2 to it
+  bool rope_small_step;       // kOutRopeI: base >= 1, so a position's step is 1 radian at most
 };
 
 struct BwdArgs {
@@ -274,10 +276,6 @@ constexpr int kOutMxE4M3 = 2;  // MXFP8: e4m3 codes, one E8M0 scale per 32 eleme
 constexpr int kOutMxE2M1 = 3;  // MXFP4: e2m1 nibbles (two per byte), one E8M0 scale per 32
 constexpr int kOutRopeI = 4;   // y rotated by the reference model's interleaved RoPE
 constexpr int kOutDtypeLateH = 5;  // as kOutDtype, with h stored after the row reduction
-// y rotated by the interleaved RoPE with each pair's (cos, sin) evaluated directly: rows too wide
-// for fwd_rope_kernel's walk (more than one 16-byte chunk per thread)
-constexpr int kOutRopeDirect = 6;
-
 // The reference model's RoPE applied to y in registers (python/velograd/functional.py:287-315;
 // models/llama.py:48-49 rotates the normalised attention input): the pair (y_2i, y_2i+1) of a
 // row at position pos turns by pos * freq_i, freq_i = base^(-2i/dim) = 2^-(i * c) with
@@ -287,6 +285,7 @@ constexpr int kOutRopeDirect = 6;
 // a few float32 ulps at any position (a float32 angle would carry pos * freq_i * 2^-24 radians of
 // error: 0.016 rad at position 2.6e5).
 constexpr double kInv2PiD = 0.159154943091895335768883763372514362;
+constexpr double kTwoPiD = 6.283185307179586476925286766559005768;
 __device__ __forceinline__ double rope_freq(int i, float c_hi, float c_lo) {
   return exp2(-(double)i * ((double)c_hi + (double)c_lo));
 }
@@ -320,6 +319,87 @@ struct RopeFreqWalk {
 __device__ __forceinline__ void rope_cos_sin_f(int64_t pos, double fr, float& c, float& s) {
   const double rev = (double)pos * fr * kInv2PiD;
   sincospif(2.0f * (float)(rev - rint(rev)), &s, &c);
+}
+
+// A double angle in revolutions reduced exactly to [-1/2, 1/2], and the cos and sin of such an
+// angle: the quarter turn nearest to it, then the Taylor series of sin and cos over the +-1/8
+// turn that is left (0.72 and 0.98 ulp at most against 64 bits over 4 million angles; the leading
+// pi/2 in two floats).
+__device__ __forceinline__ float rope_frac(double rev) { return (float)(rev - rint(rev)); }
+__device__ __forceinline__ void cos_sin_turn(float rev, float& c, float& s) {
+  const float t = 4.0f * rev;
+  const float k = rintf(t);
+  const float f = t - k;  // quarter turns, exact
+  const float z = f * f;
+  float ps = 0.00016044118478735975f;  // (pi/2)^n / n!, alternating
+  ps = fmaf(ps, z, -0.004681754135318687f);
+  ps = fmaf(ps, z, 0.07969262624616703f);
+  ps = fmaf(ps, z, -0.6459640975062462f);
+  ps = fmaf(ps, z, -4.371139000186241e-8f);  // pi/2 - (float)(pi/2)
+  const float s0 = fmaf(f, 1.5707963267948966f, f * ps);
+  float pc = -2.5202042373060596e-05f;
+  pc = fmaf(pc, z, 0.0009192602748394263f);
+  pc = fmaf(pc, z, -0.020863480763352957f);
+  pc = fmaf(pc, z, 0.253669507901048f);
+  pc = fmaf(pc, z, -1.2337005501361697f);
+  const float c0 = fmaf(pc, z, 1.0f);
+  const int q = (int)k;
+  const bool odd = (q & 1) != 0;
+  s = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, odd ? c0 : s0) ^
+                                    ((uint32_t)(q & 2) << 30));
+  c = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, odd ? s0 : c0) ^
+                                    ((uint32_t)((q + 1) & 2) << 30));
+}
+
+// cos and sin of |x| <= 1 in double by their Taylor series through x^14 and x^13 (truncation below
+// 1e-12).
+__device__ __forceinline__ void cos_sin_small_d(double x, double& c, double& s) {
+  const double z = x * x;
+  double ps = 1.0 / 6227020800.0;
+  ps = fma(ps, z, -1.0 / 39916800.0);
+  ps = fma(ps, z, 1.0 / 362880.0);
+  ps = fma(ps, z, -1.0 / 5040.0);
+  ps = fma(ps, z, 1.0 / 120.0);
+  ps = fma(ps, z, -1.0 / 6.0);
+  s = fma(x * z, ps, x);
+  double pc = -1.0 / 87178291200.0;
+  pc = fma(pc, z, 1.0 / 479001600.0);
+  pc = fma(pc, z, -1.0 / 3628800.0);
+  pc = fma(pc, z, 1.0 / 40320.0);
+  pc = fma(pc, z, -1.0 / 720.0);
+  pc = fma(pc, z, 1.0 / 24.0);
+  pc = fma(pc, z, -0.5);
+  c = fma(z, pc, 1.0);
+}
+
+// cos and sin of 2 pi rev in double, |rev| <= 1/2: Taylor series of an eighth of the angle
+// (|x| <= pi/8: truncation below 1e-17), doubled three times.
+__device__ __forceinline__ void cos_sin_turn_d(double rev, double& c, double& s) {
+  const double x = rev * 0.78539816339744830961566084581987572;  // 2 pi / 8
+  const double z = x * x;
+  double ps = -1.0 / 1307674368000.0;
+  ps = fma(ps, z, 1.0 / 6227020800.0);
+  ps = fma(ps, z, -1.0 / 39916800.0);
+  ps = fma(ps, z, 1.0 / 362880.0);
+  ps = fma(ps, z, -1.0 / 5040.0);
+  ps = fma(ps, z, 1.0 / 120.0);
+  ps = fma(ps, z, -1.0 / 6.0);
+  s = fma(x * z, ps, x);
+  double pc = 1.0 / 20922789888000.0;  // cos x - 1
+  pc = fma(pc, z, -1.0 / 87178291200.0);
+  pc = fma(pc, z, 1.0 / 479001600.0);
+  pc = fma(pc, z, -1.0 / 3628800.0);
+  pc = fma(pc, z, 1.0 / 40320.0);
+  pc = fma(pc, z, -1.0 / 720.0);
+  pc = fma(pc, z, 1.0 / 24.0);
+  pc = fma(pc, z, -0.5);
+  pc = pc * z;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {  // v = cos - 1: v(2x) = 2 v (2 + v), sin(2x) = 2 sin (1 + v)
+    s = 2.0 * fma(s, pc, s);
+    pc = 2.0 * pc * (2.0 + pc);
+  }
+  c = 1.0 + pc;
 }
 
 // Largest value over aligned groups of L lanes (L = 4 or 8), on every lane of the group.
@@ -363,7 +443,6 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
   using C = Codec<DT>;
   constexpr int V = C::kVec;
   constexpr bool ANY = ROWS != kRowsChunks;
-  static_assert(!ANY || OUT != kOutRopeDirect, "the RoPE output takes aligned rows here");
   __shared__ float red[kMaxWavesPerRow];
 
   const int tpr = a.tpr;
@@ -498,8 +577,8 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
     for (int i = 0; i < V; ++i) yf[i] = (hf[i] * r) * wf[i];
   };
 
-  static_assert(OUT != kOutRopeI, "the RoPE output runs in fwd_rope_kernel");
-  if constexpr (OUT == kOutDtype || OUT == kOutDtypeLateH || OUT == kOutRopeDirect) {
+  static_assert(OUT != kOutRopeI, "the RoPE output runs in fwd_rope_tile_kernel");
+  if constexpr (OUT == kOutDtype || OUT == kOutDtypeLateH) {
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       const int c = lt + k * tpr;
@@ -511,20 +590,6 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
         }
         float yf[V];
         make_y(k, yf);
-        if constexpr (OUT == kOutRopeDirect) {
-          // pairs c * V/2 + q at position row % rope_seq (functional.py:302-314): double
-          // frequency and angle, exact reduction, float sincospi, as rope_cos_sin
-          const int64_t pos = row % a.rope_seq;
-          RopeFreqWalk fw(c * (V / 2), 1, a.rope_c_hi, a.rope_c_lo);
-#pragma unroll
-          for (int q = 0; q < V / 2; ++q) {
-            float cs, sn;
-            rope_cos_sin_f(pos, fw.next(), cs, sn);
-            const float y0 = yf[2 * q], y1 = yf[2 * q + 1];
-            yf[2 * q] = y0 * cs - y1 * sn;                                 // functional.py:313
-            yf[2 * q + 1] = y0 * sn + y1 * cs;                             // functional.py:314
-          }
-        }
         store_chunk(a.y, row * a.ld_y + col_of(c), C::pack(yf));
       }
     }
@@ -631,225 +696,231 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
 }
 
 // ------------------------------------------------------------------------------------------
-// Forward with the model's RoPE on y (kOutRopeI), one 16-byte chunk per thread.  Workgroup b of
-// G walks up to W rows b, b + G, b + 2G, ... (W = 16, or 32 for long tensors of wide rows:
-// launch_plan.h fwd_rope_walk_rows): at each step the resident workgroups
-// touch adjacent rows, one compact address front that HBM serves better than runs of
-// consecutive rows per workgroup (those spread the front over 16 rows per workgroup).  The next
-// rows' chunks are in flight while the current one reduces.  Each thread keeps the rotation
-// (cos, sin) of its pairs (in double for fp32 outputs, in float32 for bf16/fp16 ones) and
-// advances it by G positions per step (the rotation through G * freq_j, evaluated once per walk),
-// so trigonometry runs only before the walk; evaluated per (row, pair) it made the fused pass
-// VALU-bound, no faster than two passes.  The walk's first angle is the double pos * freq_j
-// reduced exactly before a float sincospi (a few float32 ulps), and so is the step's; the
-// recurrence adds ~1e-16 per step in double, about 3 float32 ulps of the pair in float32, over
-// at most W - 1 steps from an exact value.  Where a step crosses
-// the end of a sequence (row position = row % rope_seq) and G is a multiple or a divisor of
-// rope_seq, the position returns to the walk's first one and so does the rotation (kept); any
-// other crossing re-evaluates the angle at the new position.
-// The pass is bound by its vector instructions as much as by HBM, so each row's arithmetic is
-// kept short: the weight is decoded once per walk, h stays in registers across the reduction,
-// sums of products and the rotation use fused multiply-adds, and for a power-of-two dim the mean
-// is sum * (1 / dim), exact, instead of a division.
-// A whole walk whose positions only advance or return to the start (the usual case) runs as
-// straight-line code over its rows with a ring of three row buffers, two rows' loads in flight
-// while one reduces, and no branch around a global memory operation (the residual and h are
-// compile-time flags RF; the walk's inv_rms values wait in LDS and are stored after it), so
-// each row waits for its own loads only instead of draining every load and store at each row.
-// Shorter walks and walks that re-evaluate angles take the guarded loop.
+// Forward with the model's RoPE on y (kOutRopeI): a one-shot grid of tiles.  A row group takes R
+// consecutive positions of one sequence (a position past the sequence's end re-reads the last one
+// and stores nothing): all their loads are in flight at once, the rotations are formed while they
+// are, one barrier serves the R row sums, and consecutive tiles run on one XCD (xcd_item).
+// Angles, as the reference's Python floats form them (functional.py:302-305): pair j turns
+// g_j = base^(-2j/dim) / (2 pi) revolutions per position, in double (one exp2 per chunk, its next
+// pairs by the double ratio); the tile's first position times g_j in double is reduced exactly to
+// [-1/2, 1/2] revolutions before a float cos and sin (cos_sin_turn), and the next positions
+// advance that by the step rotation, at most R - 1 times: in float for bf16/fp16 outputs (3
+// float32 ulps a step at most, far below their rounding), in double for fp32 ones.
+// Short tiles cost trigonometry, which the vector units pay (28 instructions an element at four
+// positions), long ones parallelism; a walk of 16 or 32 strided rows per workgroup instead, its
+// trigonometry set up once, left most of the chip idle on short tensors and waited at every row.
+// Measured (bf16 without residual, that walk / tiles, us): 64 x 4096 16.0 / 3.5, 2048 x 4096 16.7 /
+// 8.1, 8192 x 4096 26.9 / 25.4, 16384 x 4096 49.8 / 45.9 (the norm alone 43.7), 16384 x 768 18.6 /
+// 11.4, 8192 x 8192 52.1 / 49.9, fp32 8192 x 4096 49.4 / 49.8; with residual and h 16384 x 4096
+// 97.4 / 88.2.  Rows of two chunks a thread, whose pairs were each evaluated at every row:
+// 8192 x 16384 160 / 111, fp32 8192 x 8192 133 / 107.  Error against 64 bits in fp32: 8.1e-8 both.
+// ANY: even rows that are not whole chunks, streams at any element: the row's last chunk begins at
+// dim - V, inside the one before it; the columns it shares add nothing and are not stored (4100
+// bf16, generic kernel / tiles, 8192 rows: 100 / 28.6 us; 3002 74 / 21.5; 1000, aligned, 16.8 / 7.5).
 // ------------------------------------------------------------------------------------------
-constexpr int kRopeRes = 1;     // RF: a residual is added
-constexpr int kRopeWriteH = 2;  // RF: h is stored
-constexpr int kRopeDimPow2 = 4; // RF: dim is a power of two
-
-template <int DT, int WDT, int RF, int W>
-__global__ __launch_bounds__(max_block_for_nv(1)) void fwd_rope_kernel(const FwdArgs a) {
-  static_assert(W == vg_plan::kNormRopeRows || W == vg_plan::kNormRopeLongRows,
-                "walks of 16 or 32 rows");
+template <int DT, int WDT, int NV, bool RES, int R, bool ANY>
+__global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_rope_tile_kernel(const FwdArgs a) {
   using C = Codec<DT>;
   constexpr int V = C::kVec;
-  constexpr int PP = V / 2;  // pairs per chunk
-  __shared__ float red[2][kMaxWavesPerRow];
-  const int tpr = blockDim.x;  // one row group per workgroup, one chunk per thread
-  const int lt = threadIdx.x;
-  const int nchunk = a.dim / V;
-  const bool lane_ok = lt < nchunk;
-  constexpr bool has_res = (RF & kRopeRes) != 0;
-  constexpr bool write_h = has_res && (RF & kRopeWriteH) != 0;
+  constexpr int P = V / 2;     // pairs per chunk
+  constexpr int NP = NV * P;   // pairs per thread
+  constexpr int RQ = (R + 3) / 4;  // quads of rows in the second reduction step
+  __shared__ float red[kMaxWavesPerRow][4 * RQ];
+
+  const int tpr = a.tpr;
+  const int grp = threadIdx.x / tpr;
+  const int lt = threadIdx.x - grp * tpr;
+  const int groups = blockDim.x / tpr;
+  // the tile: positions s0 .. s0 + ns - 1 of sequence o
+  const uint32_t seq = (uint32_t)a.rope_seq;
+  const uint32_t tps = (seq + R - 1) / R;
+  const uint32_t tiles = (uint32_t)(a.rows / seq) * tps;
+  const uint32_t item = xcd_item(blockIdx.x, gridDim.x, a.run_log2) * groups + grp;
+  const bool ok = item < tiles;
+  const uint32_t tile = ok ? item : tiles - 1;
+  const uint32_t o = tile / tps;
+  const uint32_t s0 = (tile - o * tps) * R;
+  const int ns = (int)min(seq - s0, (uint32_t)R);
+  const int64_t row0 = (int64_t)o * seq + s0;
   const bool has_w = a.w != nullptr;
-  const int64_t G = gridDim.x;   // row step of the walk
-  const int64_t row0 = blockIdx.x;
-  const int64_t left = (a.rows - row0 + G - 1) / G;
-  const int nrows = (int)(left < W ? left : W);
-  const int64_t col = (int64_t)lt * V;
-  const int64_t seq = a.rope_seq;
-  const int64_t pos0 = row0 % seq;
-  // the positions of the walk only advance by G or return to pos0
-  const bool back_to_start = (seq % G == 0) || (G % seq == 0);
-  // 1 / dim is exact for a power of two, so sum * (1 / dim) has the bits of sum / dim
-  const float inv_dim = (RF & kRopeDimPow2) ? 1.0f / (float)a.dim : 0.0f;
-
-  u32x4 xv = u32x4{0u, 0u, 0u, 0u}, rv = u32x4{0u, 0u, 0u, 0u};
-  if (lane_ok) {
-    xv = load16_stream<DT>(a.x, row0 * a.ld_x + col);
-    if constexpr (has_res) rv = load16_stream<DT>(a.res, row0 * a.ld_res + col);
-  }
-  float wf[V];
-  {
-    WeightChunk<DT, WDT> wc;
-    wc.load((has_w && lane_ok) ? a.w : nullptr, col);
-    wc.unpack(has_w, wf);
-  }
-  // The rotation state: double for fp32 outputs; float32 for bf16/fp16 ones, within about 3
-  // float32 ulps of the pair per step over at most W - 1 = 31 steps (~2^-17.5 of the pair), far
-  // below their output's rounding (2^-9 for bf16, 2^-12 for fp16).  Re-evaluating it at the 16th
-  // row of a 32-row walk cost 2-5 us at 16384 rows (trigonometry set aside for it before the
-  // walk; placed in the unrolled loop it stopped the unrolling).
-  using RotT = std::conditional_t<DT == VELOGRAD_DTYPE_F32, double, float>;
-  auto rot_fma = [](RotT x, RotT y, RotT z) {
-    if constexpr (DT == VELOGRAD_DTYPE_F32) return __builtin_fma(x, y, z);
-    else return __builtin_fmaf(x, y, z);
-  };
-  RotT cr[PP], sr[PP], cst[PP], sst[PP];
-  float c0[PP], s0[PP];  // the rotation at pos0
-  // the rotation at pos: double angle, reduced exactly, float sincospi
-  auto rotation_at = [&](int64_t pos, int q, float& c, float& s) {
-    const double rev = (double)pos * rope_freq(lt * PP + q, a.rope_c_hi, a.rope_c_lo) * kInv2PiD;
-    sincospif(2.0f * (float)(rev - rint(rev)), &s, &c);
-  };
+  const int nchunk = ANY ? (a.dim + V - 1) / V : a.dim / V;
+  int col[NV];    // first column of the lane's chunks
+  bool own[NV];
 #pragma unroll
-  for (int q = 0; q < PP; ++q) {
-    // the rotation through G positions: double for fp32 outputs, else as rotation_at
-    if constexpr (DT == VELOGRAD_DTYPE_F32) {
-      double sv, cv;
-      sincos((double)G * rope_freq(lt * PP + q, a.rope_c_hi, a.rope_c_lo), &sv, &cv);
-      cst[q] = cv;
-      sst[q] = sv;
-    } else {
-      float sv, cv;
-      rotation_at(G, q, cv, sv);
-      cst[q] = cv;
-      sst[q] = sv;
-    }
-    rotation_at(pos0, q, c0[q], s0[q]);
-    cr[q] = c0[q];
-    sr[q] = s0[q];
+  for (int k = 0; k < NV; ++k) {
+    const int c = lt + k * tpr;
+    own[k] = c < nchunk;
+    col[k] = min(c * V, a.dim - V);
   }
 
-  auto make_h = [&](const u32x4& xq, const u32x4& rq, float* hf) {
-    C::unpack(xq, hf);
-    if constexpr (has_res) {
+  u32x4 xv[R][NV], rv[RES ? R : 1][NV];
+  WeightChunk<DT, WDT> wc[NV];
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    const int64_t row = row0 + (u < ns ? u : ns - 1);
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      if constexpr (ANY) {
+        xv[u][k] = load16_any_stream<DT>(a.x, row * a.ld_x + col[k]);
+        if constexpr (RES) rv[u][k] = load16_any_stream<DT>(a.res, row * a.ld_res + col[k]);
+      } else {
+        xv[u][k] = load16_stream<DT>(a.x, row * a.ld_x + col[k]);
+        if constexpr (RES) rv[u][k] = load16_stream<DT>(a.res, row * a.ld_res + col[k]);
+      }
+    }
+  }
+  if (has_w) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      if constexpr (ANY) wc[k].load_any(a.w, col[k]);
+      else wc[k].load(a.w, col[k]);
+    }
+  }
+
+  // the rotation of each pair at s0 and its step, while the loads are in flight
+  using RotT = std::conditional_t<DT == VELOGRAD_DTYPE_F32, double, float>;
+  RotT cr[NP], sr[NP], cs[NP], sn[NP];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    double g = exp2((double)(col[k] / 2) * a.rope_log2_step) * kInv2PiD;  // revolutions a position
+#pragma unroll
+    for (int q = 0; q < P; ++q) {
+      const int e = k * P + q;
+      float c0, s0f;
+      cos_sin_turn(rope_frac((double)s0 * g), c0, s0f);
+      cr[e] = c0;
+      sr[e] = s0f;
+      if constexpr (R > 1) {
+        if constexpr (DT == VELOGRAD_DTYPE_F32) {
+          if (a.rope_small_step) cos_sin_small_d(g * kTwoPiD, cs[e], sn[e]);
+          else cos_sin_turn_d(g - rint(g), cs[e], sn[e]);
+        } else {
+          if (a.rope_small_step) cos_sin_small((float)(g * kTwoPiD), cs[e], sn[e]);
+          else cos_sin_turn(rope_frac(g), cs[e], sn[e]);
+        }
+      }
+      g *= a.rope_ratio;
+    }
+  }
+
+  auto make_h = [&](int u, int k, float* hf) {
+    C::unpack(xv[u][k], hf);
+    if constexpr (RES) {
       float rf[V];
-      C::unpack(rq, rf);
+      C::unpack(rv[u][k], rf);
 #pragma unroll
       for (int i = 0; i < V; ++i) hf[i] = hf[i] + rf[i];
     }
   };
-  auto sum_sq = [&](const float* hf) {
+  // ANY: the row's last chunk may begin inside the one before it; those columns are not its own
+  auto skip_of = [&](int k) { return ANY ? (lt + k * tpr) * V - col[k] : 0; };
+
+  // row sums: each wave's in its lane 0, then the waves' of four rows at once, one row to each
+  // 16 lanes
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
     float ss = 0.0f;
 #pragma unroll
-    for (int i = 0; i < V; ++i) ss = __builtin_fmaf(hf[i], hf[i], ss);
-    return ss;
-  };
-  auto inv_rms_of = [&](float ss) {
-    const float mean = (RF & kRopeDimPow2) ? ss * inv_dim : ss / (float)a.dim;
-    return 1.0f / __builtin_sqrtf(floor_mean_sq(mean, a.ms_floor) + a.eps);
-  };
-  // y = (h * r) * w turned by the current angles
-  auto make_y = [&](const float* hf, float r, float* yf) {
-#pragma unroll
-    for (int i = 0; i < V; ++i) yf[i] = (hf[i] * r) * wf[i];
-#pragma unroll
-    for (int q = 0; q < PP; ++q) {
-      const float cv = (float)cr[q], sv = (float)sr[q];
-      const float y0 = yf[2 * q], y1 = yf[2 * q + 1];
-      yf[2 * q] = __builtin_fmaf(y0, cv, -(y1 * sv));                    // functional.py:313
-      yf[2 * q + 1] = __builtin_fmaf(y0, sv, y1 * cv);                   // functional.py:314
-    }
-  };
-  // the angles of the next row of the walk: pos advances by G; past the end of the sequence it
-  // returns to pos0 (back_to_start) or, with ANCHOR, lands anywhere and is evaluated afresh
-  auto advance = [&](int64_t& pos, auto anchor) {
-    pos += G;
-    if (pos < seq) {
-#pragma unroll
-      for (int q = 0; q < PP; ++q) {
-        const RotT cn = rot_fma(cr[q], cst[q], -(sr[q] * sst[q]));
-        sr[q] = rot_fma(sr[q], cst[q], cr[q] * sst[q]);
-        cr[q] = cn;
-      }
-    } else if (!decltype(anchor)::value || back_to_start) {
-      pos = pos0;
-#pragma unroll
-      for (int q = 0; q < PP; ++q) {
-        cr[q] = c0[q];
-        sr[q] = s0[q];
-      }
-    } else {
-      pos %= seq;
-#pragma unroll
-      for (int q = 0; q < PP; ++q) {
-        float c, s;
-        rotation_at(pos, q, c, s);
-        cr[q] = c;
-        sr[q] = s;
-      }
-    }
-  };
-
-  const bool walk_ok = back_to_start || pos0 + (int64_t)(W - 1) * G < seq;
-  if (nrows == W && nchunk == tpr && walk_ok) {
-    __shared__ float inv_lds[W];
-    constexpr int RB = 3;
-    u32x4 xb[RB], rb[RB];
-    xb[0] = xv;
-    rb[0] = rv;
-    xb[1] = load16_stream<DT>(a.x, (row0 + G) * a.ld_x + col);
-    if constexpr (has_res) rb[1] = load16_stream<DT>(a.res, (row0 + G) * a.ld_res + col);
-    int64_t pos = pos0;
-#pragma unroll
-    for (int it = 0; it < W; ++it) {
-      const int b = it % RB;
-      const int64_t row = row0 + it * G;
-      if (it + 2 < W) {
-        const int nb = (it + 2) % RB;
-        xb[nb] = load16_stream<DT>(a.x, (row + 2 * G) * a.ld_x + col);
-        if constexpr (has_res) rb[nb] = load16_stream<DT>(a.res, (row + 2 * G) * a.ld_res + col);
-      }
+    for (int k = 0; k < NV; ++k) {
       float hf[V];
-      make_h(xb[b], rb[b], hf);
-      if constexpr (write_h) store16_stream<DT>(a.h, row * a.ld_h + col, C::pack(hf));
-      const float r = inv_rms_of(row_sum(sum_sq(hf), tpr, 0, red[it & 1]));
-      if (lt == 0) inv_lds[it] = r;
-      float yf[V];
-      make_y(hf, r, yf);
-      store16_stream<DT>(a.y, row * a.ld_y + col, C::pack(yf));
-      if (it + 1 < W) advance(pos, std::false_type{});
+      make_h(u, k, hf);
+      float p = 0.0f;
+      if constexpr (ANY) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+          const float t = i >= skip_of(k) ? hf[i] : 0.0f;
+          p = __builtin_fmaf(t, t, p);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < V; ++i) p = __builtin_fmaf(hf[i], hf[i], p);
+      }
+      ss += own[k] ? p : 0.0f;
     }
-    // thread 0 wrote inv_lds; threads 1..W-1 of its wave read it in program order
-    if (lt < W && a.inv_rms != nullptr) a.inv_rms[row0 + lt * G] = inv_lds[lt];
-    return;
+    ss = wave_sum(ss);
+    if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave][u] = ss;
+  }
+  __syncthreads();
+  float r[R];
+  {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wpr = tpr / kWave;
+    const int w = lane & 15;
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) {
+      const int u = 4 * q + (lane >> 4);
+      float t = (w < wpr && u < R) ? red[grp * wpr + (w < wpr ? w : 0)][u] : 0.0f;
+      t += dpp_move<0xB1>(t);
+      t += dpp_move<0x4E>(t);
+      t += dpp_move<0x124>(t);
+      t += dpp_move<0x128>(t);
+      const float mean = t / (float)a.dim;
+      const float ir = 1.0f / __builtin_sqrtf(floor_mean_sq(mean, a.ms_floor) + a.eps);
+      if (lt < kWave && w == 0 && ok && u < ns && a.inv_rms != nullptr) a.inv_rms[row0 + u] = ir;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (4 * q + j < R)
+          r[4 * q + j] = __builtin_bit_cast(
+              float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ir), 16 * j));
+      }
+    }
   }
 
-  int64_t pos = pos0;
-  for (int it = 0; it < nrows; ++it) {
-    const int64_t row = row0 + it * G;
-    u32x4 xn = u32x4{0u, 0u, 0u, 0u}, rn = u32x4{0u, 0u, 0u, 0u};
-    if (it + 1 < nrows && lane_ok) {
-      xn = load16_stream<DT>(a.x, (row + G) * a.ld_x + col);
-      if constexpr (has_res) rn = load16_stream<DT>(a.res, (row + G) * a.ld_res + col);
+  const bool write_h = RES && a.h != nullptr;
+  float wf[NV][V];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) wc[k].unpack(has_w, wf[k]);
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    const int64_t row = row0 + u;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      float hf[V];
+      forget(xv[u][k]);
+      if constexpr (RES) forget(rv[u][k]);
+      make_h(u, k, hf);
+      const bool store = ok && u < ns && own[k];
+      auto put = [&](void* base, int64_t ld, const u32x4 v) {
+        if (!store) return;
+        if constexpr (ANY) {
+          const int skip = skip_of(k);
+          if (skip == 0) {
+            store16_any_stream<DT>(base, row * ld + col[k], v);
+          } else {
+#pragma unroll
+            for (int i = 2; i < V; ++i) {
+              if (i >= skip) {
+                float f[V];
+                C::unpack(v, f);
+                C::store1(base, row * ld + col[k] + i, f[i]);
+              }
+            }
+          }
+        } else {
+          store16_stream<DT>(base, row * ld + col[k], v);
+        }
+      };
+      if (write_h) put(a.h, a.ld_h, C::pack(hf));
+      float yf[V];
+#pragma unroll
+      for (int i = 0; i < V; ++i) yf[i] = (hf[i] * r[u]) * wf[k][i];
+#pragma unroll
+      for (int q = 0; q < P; ++q) {
+        const int e = k * P + q;
+        const float c = (float)cr[e], s = (float)sr[e];
+        if constexpr (R > 1) {
+          if (u + 1 < R) {
+            const RotT cn = __builtin_elementwise_fma(cr[e], cs[e], -(sr[e] * sn[e]));
+            sr[e] = __builtin_elementwise_fma(sr[e], cs[e], cr[e] * sn[e]);
+            cr[e] = cn;
+          }
+        }
+        const float y0 = yf[2 * q], y1 = yf[2 * q + 1];
+        yf[2 * q] = __builtin_fmaf(y0, c, -(y1 * s));                      // functional.py:313
+        yf[2 * q + 1] = __builtin_fmaf(y0, s, y1 * c);                     // functional.py:314
+      }
+      put(a.y, a.ld_y, C::pack(yf));
     }
-    float hf[V];
-    make_h(xv, rv, hf);
-    if (write_h && lane_ok) store16_stream<DT>(a.h, row * a.ld_h + col, C::pack(hf));
-    const float r = inv_rms_of(row_sum(sum_sq(hf), tpr, 0, red[it & 1]));
-    if (lt == 0 && a.inv_rms != nullptr) a.inv_rms[row] = r;
-    float yf[V];
-    make_y(hf, r, yf);
-    if (lane_ok) store16_stream<DT>(a.y, row * a.ld_y + col, C::pack(yf));
-    if (it + 1 < nrows) advance(pos, std::true_type{});
-    xv = xn;
-    rv = rn;
   }
 }
 
@@ -2539,51 +2610,7 @@ void launch_fwd(const FwdArgs& a, const RowPlan& p, hipStream_t st) {
                        0, st, a);
     return;
   }
-  if constexpr (OUT == kOutRopeI) {
-    // One chunk per thread (rows up to 1024 chunks: 8192 bf16/fp16, 4096 fp32 elements); more
-    // chunks would hold 16 more doubles per chunk and spill, so longer rows take the generic
-    // kernel.
-    if (p.nv != 1) {
-      // wider rows: the register-resident one-shot rows with each pair's rotation evaluated
-      // directly (1024-thread row groups, two to four chunks per thread)
-      const dim3 grid((uint32_t)((a.rows + p.groups - 1) / p.groups)), block(p.block);
-      switch (p.nv) {
-        case 2:
-          hipLaunchKernelGGL((fwd_vec_kernel<DT, WDT, 2, kOutRopeDirect>), grid, block, 0, st, a);
-          break;
-        case 3:
-          hipLaunchKernelGGL((fwd_vec_kernel<DT, WDT, 3, kOutRopeDirect>), grid, block, 0, st, a);
-          break;
-        default:
-          hipLaunchKernelGGL((fwd_vec_kernel<DT, WDT, 4, kOutRopeDirect>), grid, block, 0, st, a);
-          break;
-      }
-      return;
-    }
-    const int w = vg_plan::fwd_rope_walk_rows(a.rows, p.tpr);
-    const dim3 grid((uint32_t)((a.rows + w - 1) / w)), block(p.tpr);
-    const int rf = (a.res == nullptr ? 0 : a.h == nullptr ? kRopeRes : kRopeRes | kRopeWriteH) |
-                   ((a.dim & (a.dim - 1)) == 0 ? kRopeDimPow2 : 0);
-    switch (rf * 2 + (w == vg_plan::kNormRopeLongRows ? 1 : 0)) {
-#define VG_ROPE_FWD(F)                                                                      \
-  case 2 * (F):                                                                             \
-    hipLaunchKernelGGL((fwd_rope_kernel<DT, WDT, F, vg_plan::kNormRopeRows>), grid, block, 0, \
-                       st, a);                                                              \
-    break;                                                                                  \
-  case 2 * (F) + 1:                                                                         \
-    hipLaunchKernelGGL((fwd_rope_kernel<DT, WDT, F, vg_plan::kNormRopeLongRows>), grid,       \
-                       block, 0, st, a);                                                    \
-    break;
-      VG_ROPE_FWD(0)
-      VG_ROPE_FWD(kRopeRes)
-      VG_ROPE_FWD(kRopeRes | kRopeWriteH)
-      VG_ROPE_FWD(kRopeDimPow2)
-      VG_ROPE_FWD(kRopeDimPow2 | kRopeRes)
-      VG_ROPE_FWD(kRopeDimPow2 | kRopeRes | kRopeWriteH)
-#undef VG_ROPE_FWD
-      default: break;
-    }
-  } else {
+  if constexpr (OUT != kOutRopeI) {  // (the RoPE output's rows run in fwd_rope_tile_kernel)
     const dim3 grid((uint32_t)((a.rows + p.groups - 1) / p.groups));
     const dim3 block(p.block);
     if constexpr (OUT == kOutDtype) {
@@ -2632,6 +2659,37 @@ template <int DT, int WDT, int OUT>
 void launch_fwd_any(const FwdArgs& a, const RowPlan& p, hipStream_t st) {
   if (a.res != nullptr) launch_fwd_any_rows<DT, WDT, OUT, kRowsAnyRes>(a, p, st);
   else launch_fwd_any_rows<DT, WDT, OUT, kRowsAnyNoRes>(a, p, st);
+}
+
+// The norm + RoPE tiles (vg_plan::RopeTilePlan).
+template <int DT, int WDT, int NV, bool RES, bool ANY>
+void launch_rope_tile(const FwdArgs& a, const vg_plan::RopeTilePlan& p, hipStream_t st) {
+  const dim3 grid((uint32_t)p.wgs), block(p.rp.block);
+  if constexpr (!RES) {
+    if (p.tile == 4) {
+      hipLaunchKernelGGL((fwd_rope_tile_kernel<DT, WDT, NV, RES, 4, ANY>), grid, block, 0, st, a);
+      return;
+    }
+  }
+  if (p.tile == 2)
+    hipLaunchKernelGGL((fwd_rope_tile_kernel<DT, WDT, NV, RES, 2, ANY>), grid, block, 0, st, a);
+  else
+    hipLaunchKernelGGL((fwd_rope_tile_kernel<DT, WDT, NV, RES, 1, ANY>), grid, block, 0, st, a);
+}
+
+template <int DT, int WDT>
+void launch_rope_tiles(const FwdArgs& a, const vg_plan::RopeTilePlan& p, bool any, hipStream_t st) {
+  const int which = (p.rp.nv == 2 ? 4 : 0) | (a.res != nullptr ? 2 : 0) | (any ? 1 : 0);
+  switch (which) {
+    case 0: launch_rope_tile<DT, WDT, 1, false, false>(a, p, st); break;
+    case 1: launch_rope_tile<DT, WDT, 1, false, true>(a, p, st); break;
+    case 2: launch_rope_tile<DT, WDT, 1, true, false>(a, p, st); break;
+    case 3: launch_rope_tile<DT, WDT, 1, true, true>(a, p, st); break;
+    case 4: launch_rope_tile<DT, WDT, 2, false, false>(a, p, st); break;
+    case 5: launch_rope_tile<DT, WDT, 2, false, true>(a, p, st); break;
+    case 6: launch_rope_tile<DT, WDT, 2, true, false>(a, p, st); break;
+    default: launch_rope_tile<DT, WDT, 2, true, true>(a, p, st); break;
+  }
 }
 
 // Rows of element-strided lanes (fwd_elem_kernel): `p` from plan_elem_rows, m elements a lane.
@@ -2885,7 +2943,7 @@ int32_t run_fwd(const char* what, int out, const void* x, const void* residual,
   const int eb = elem_bytes_of(dtype);
   // Bytes of y per 16-byte input chunk: 16 (activation dtype), 16 / eb (e4m3), 8 / eb (e2m1).
   bool y_aligned;
-  if (out == kOutDtype) {
+  if (out == kOutDtype || out == kOutRopeI) {
     y_aligned = aligned16(y) && ld_ok(ld_y, eb);
   } else {
     const int64_t cb = out == kOutMxE2M1 ? 8 / eb : 16 / eb;
@@ -2894,12 +2952,11 @@ int32_t run_fwd(const char* what, int out, const void* x, const void* residual,
   const bool aligned = aligned16(x) && ld_ok(ld_x, eb) && y_aligned &&
                        (!residual || (aligned16(residual) && ld_ok(ld_res, eb))) &&
                        (!h || (aligned16(h) && ld_ok(ld_h, eb))) && (!weight || aligned16(weight));
-  // The fused norm + RoPE kernel holds one chunk per thread, so it keeps the residual order
-  // (one chunk first) either way.
-  RowPlan p = plan_fwd(dim, eb, aligned, residual == nullptr && out != kOutRopeI,
+  RowPlan p = plan_fwd(dim, eb, aligned && out != kOutRopeI, residual == nullptr,
                        out == kOutFp8Row || mx);
   // rows the chunked layout does not fit, on element boundaries
-  const bool aligned_elem = elem_ok_ptr(x, eb) && (out != kOutDtype || elem_ok_ptr(y, eb)) &&
+  const bool aligned_elem = elem_ok_ptr(x, eb) &&
+                            ((out != kOutDtype && out != kOutRopeI) || elem_ok_ptr(y, eb)) &&
                             elem_ok_ptr(residual, eb) && elem_ok_ptr(h, eb) &&
                             elem_ok_ptr(weight, elem_bytes_of(w_dtype));
   // The shortest of them go element by element, several rows a workgroup; the others in chunks
@@ -2955,7 +3012,21 @@ int32_t run_fwd(const char* what, int out, const void* x, const void* residual,
                                                    : 0.0;
   a.rope_c_hi = (float)c;
   a.rope_c_lo = (float)(c - (double)a.rope_c_hi);
+  a.rope_log2_step = -c;
+  a.rope_ratio = exp2(-c);
+  a.rope_small_step = rope_theta >= 1.0f;
   hipStream_t st = static_cast<hipStream_t>(hip_stream);
+  if (out == kOutRopeI && aligned_elem) {
+    const vg_plan::RopeTilePlan t =
+        vg_plan::plan_rope_tiles(rows, dim, eb, rope_seq, residual != nullptr);
+    if (t.rp.vec) {
+      a.tpr = t.rp.tpr;
+      a.run_log2 = vg_plan::xcd_run_log2(dim * eb * t.tile, t.rp.groups);
+      const bool any = !aligned || dim % (16 / eb) != 0;
+      VG_DISPATCH_TYPES(dtype, w_dtype, (launch_rope_tiles<kD, kW>(a, t, any, st)));
+      return check_launch(what);
+    }
+  }
   switch (out) {
 #define VG_FWD_OUT(O)                                                                  \
   case O:                                                                              \
