@@ -214,6 +214,8 @@ struct BwdPlan {
   // the ring over rows of 8-byte alignment with a half chunk at their end (plan_bwd_ring8): rp
   // lays out the row's whole chunks (dim - 4 elements)
   bool x8 = false;
+  // the ring over rows of any length and alignment (plan_bwd_ring_any)
+  bool any = false;
   // the element-strided ring (plan_bwd_ring_elem): elements per lane, 0 when not planned
   int elem_m = 0;
   // with the RoPE gradient: bwd_vec_kernel's plain plan, each pair's rotation evaluated directly
@@ -386,6 +388,40 @@ inline BwdPlan plan_bwd_ring8(int64_t rows, int64_t dim, int elem_bytes, int cus
   }
   b.x8 = true;
   b.lds_bytes = b.rp.groups > 1 ? (size_t)dim * sizeof(float) : 0;
+  return b;
+}
+
+// The ring over rows that the chunked layout does not fit (bwd_ring_kernel's kRingAny), the row's
+// last chunk overlapping the one before it: one chunk a thread, two where that leaves a workgroup of
+// five or six waves (2503 bf16: 48.9 us, 72 element by element), for fp32 rows of more than two waves
+// (601: 26.9 against 31.9 us, 2047 72.7 against 77.2, but with grad_h 401 26.6 against 23.3) and
+// past kRingBlock chunks.
+inline BwdPlan plan_bwd_ring_any(int64_t rows, int64_t dim, int elem_bytes, int cus) {
+  BwdPlan b;
+  b.rp = RowPlan{false, 0, kGenericBlock, 1, kGenericBlock};
+  b.wgs = 0;
+  b.lds_bytes = 0;
+  if (elem_bytes != 2 && elem_bytes != 4) return b;
+  const int V = 16 / elem_bytes;
+  if (dim < V) return b;
+  const int64_t chunks = (dim + V - 1) / V;
+  const int64_t waves = (chunks + kWave - 1) / kWave;
+  const bool two = chunks > kRingBlock || waves == 5 || waves == 6 || (elem_bytes == 4 && waves > 2);
+  const int nv = two ? 2 : 1;
+  const int64_t tpr = (waves + nv - 1) / nv * kWave;
+  if (tpr > kRingBlock) return b;
+  RowPlan& p = b.rp;
+  p.vec = true;
+  p.nv = nv;
+  p.tpr = (int)tpr;
+  p.groups = kRingBlock / p.tpr;
+  p.block = p.tpr * p.groups;
+  const int64_t wgs_needed = rows > 0 ? (rows + p.groups - 1) / p.groups : 1;
+  const int64_t wgs = cus > 0 ? (int64_t)cus : 1;
+  b.wgs = wgs < wgs_needed ? wgs : wgs_needed;
+  b.lds_bytes = p.groups > 1 ? (size_t)dim * sizeof(float) : 0;
+  b.any = true;
+  b.ring = true;
   return b;
 }
 
@@ -612,6 +648,8 @@ inline size_t bwd_workspace_bytes(int64_t rows, int64_t dim, int cus, int prefer
       if (r8.ring && r8.wgs > most) most = r8.wgs;
       const BwdPlan re = plan_bwd_ring_elem(rows, dim, sizes[si], cus);
       if (re.elem_m > 0 && re.wgs > most) most = re.wgs;
+      const BwdPlan ra = plan_bwd_ring_any(rows, dim, sizes[si], cus);
+      if (ra.ring && ra.wgs > most) most = ra.wgs;
     }
   }
   return (size_t)most * (size_t)dim * sizeof(float);

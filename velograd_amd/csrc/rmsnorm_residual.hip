@@ -1535,6 +1535,7 @@ __global__ __launch_bounds__((FLAGS & kRopeG) ? vg_plan::max_block_for_nv_rope(N
 constexpr int kRingDres = 8;
 constexpr int kRingTail = 32;
 constexpr int kRing8 = 64;
+constexpr int kRingAny = 128;
 
 template <int DT, int WDT, int NV, int FLAGS>
 __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_kernel(const BwdArgs a) {
@@ -1554,6 +1555,14 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_kernel(const Bwd
   // load.  The row group is laid out over the n whole chunks.
   constexpr bool X8 = (FLAGS & kRing8) != 0;
   static_assert(!X8 || C::kBytes == 2, "rows of 8-byte alignment are of a 2-byte dtype");
+  // kRingAny: rows of any length from one chunk up whose streams start at any element.  Lane c of
+  // the row group takes the chunk at column min(c * V, dim - V), so its columns are the same in
+  // every row.  The columns that the last chunk shares with the one before it add nothing to the
+  // sums and are stored by both lanes, the same bits (one store a lane and row, as everywhere: the
+  // ring's waits count them; storing them element by element instead held the last wave up at
+  // every row, 16384 x 4095 bf16 126 us); dx must then not be grad_h itself.
+  constexpr bool ANY = (FLAGS & kRingAny) != 0;
+  static_assert(!ANY || (!X8 && !TAIL), "one row layout");
   constexpr int VH = V / 2;
   constexpr int NH = HAS_GH ? NV : 1;  // grad_h chunks (a dummy slot when absent)
   // With grad_h a third stream fills the ring: one row ahead keeps it within 256 VGPRs.
@@ -1573,14 +1582,16 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_kernel(const Bwd
   const bool has_w = a.w != nullptr;
   const int64_t last = a.rows - 1;
   // chunk k of this lane (the row's last whole one for an idle lane) and whether it is its own
-  const int nfull = a.dim / V;
-  int chunk[NV];
+  const int nfull = ANY ? (a.dim + V - 1) / V : a.dim / V;
+  int ccol[NV];  // its first column
   bool own[NV];
+  int skip[NV];  // kRingAny: its columns that are not its own to sum
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     const int c = lt + k * tpr;
-    own[k] = !TAIL || c < nfull;
-    chunk[k] = own[k] ? c : nfull - 1;
+    own[k] = !(TAIL || ANY) || c < nfull;
+    ccol[k] = ANY ? min(c * V, a.dim - V) : (own[k] ? c : nfull - 1) * V;
+    skip[k] = ANY ? (own[k] ? c * V - ccol[k] : V) : 0;
   }
   const int64_t xcol = (int64_t)a.dim - VH;  // kRing8: the extra half chunk's first column
   const bool own_x = X8 && lt == 0;
@@ -1589,7 +1600,11 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_kernel(const Bwd
   float acc[NV][V];
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    wc[k].load(has_w ? a.w : nullptr, (int64_t)chunk[k] * V);
+    if constexpr (ANY) {
+      if (has_w) wc[k].load_any(a.w, ccol[k]);
+    } else {
+      wc[k].load(has_w ? a.w : nullptr, ccol[k]);
+    }
 #pragma unroll
     for (int i = 0; i < V; ++i) acc[k][i] = 0.0f;
   }
@@ -1623,6 +1638,8 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_kernel(const Bwd
       const u32x2 lo = load8_stream<DT>(base, e);
       const u32x2 hi = load8_stream<DT>(base, e + VH);
       return u32x4{lo.x, lo.y, hi.x, hi.y};
+    } else if constexpr (ANY) {
+      return load16_any_stream<DT>(base, e);
     } else {
       return load16_stream<DT>(base, e);
     }
@@ -1631,6 +1648,8 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_kernel(const Bwd
     if constexpr (X8) {
       store8_stream<DT>(base, e, u32x2{v.x, v.y});
       store8_stream<DT>(base, e + VH, u32x2{v.z, v.w});
+    } else if constexpr (ANY) {
+      store16_any_stream<DT>(base, e, v);
     } else {
       store16_stream<DT>(base, e, v);
     }
@@ -1641,7 +1660,7 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_kernel(const Bwd
     r = a.inv_rms[rw];
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-      const int64_t col = (int64_t)chunk[k] * V;
+      const int64_t col = ccol[k];
       gv[k] = load_chunk(a.g, rw * a.ld_g + col);
       sv[k] = load_chunk(a.saved, rw * a.ld_s + col);
       if constexpr (HAS_GH) hv[k] = load_chunk(a.gh, rw * a.ld_gh + col);
@@ -1677,7 +1696,10 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_kernel(const Bwd
 #pragma unroll
       for (int i = 0; i < V; ++i) {
         gwk[k][i] = gfk[k][i] * wf[i];
-        if constexpr (TAIL) {
+        if constexpr (ANY) {
+          const float t = gwk[k][i] * xhk[k][i];
+          s += i >= skip[k] ? t : 0.0f;
+        } else if constexpr (TAIL) {
           const float t = gwk[k][i] * xhk[k][i];
           s += own[k] ? t : 0.0f;
         } else {
@@ -1704,7 +1726,7 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_kernel(const Bwd
     const float m = s / (float)a.dim;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-      const int64_t col = (int64_t)chunk[k] * V;
+      const int64_t col = ccol[k];
       const float* gf = gfk[k];
       const float* xh = xhk[k];
       float d[V];
@@ -1717,7 +1739,7 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_kernel(const Bwd
         for (int i = 0; i < V; ++i) d[i] = d[i] + ghf[i];
       }
       const u32x4 pv = C::pack(d);
-      const bool store = TAIL ? ok && own[k] : ok;
+      const bool store = (TAIL || ANY) ? ok && own[k] : ok;
       if (store) {
         store_chunk(a.dx, row * a.ld_dx + col, pv);
         if constexpr (HAS_DRES) store_chunk(a.dres, row * a.ld_dres + col, pv);
@@ -1786,10 +1808,15 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_kernel(const Bwd
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       if (!own[k]) continue;
-      const int c = chunk[k];
+      if constexpr (ANY) {
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+          if (i >= skip[k]) prow[ccol[k] + i] = acc[k][i];
+        continue;
+      }
 #pragma unroll
       for (int q = 0; q < V / 4; ++q)
-        store16<VELOGRAD_DTYPE_F32>(prow, (int64_t)c * V + 4 * q,
+        store16<VELOGRAD_DTYPE_F32>(prow, ccol[k] + 4 * q,
                                     Codec<VELOGRAD_DTYPE_F32>::pack(&acc[k][4 * q]));
     }
     if constexpr (X8) {
@@ -1803,10 +1830,11 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_kernel(const Bwd
 #pragma unroll
       for (int k = 0; k < NV; ++k) {
         if (!own[k]) continue;
-        const int c = chunk[k];
 #pragma unroll
-        for (int i = 0; i < V; ++i)
-          comb[c * V + i] = (gi == 0) ? acc[k][i] : comb[c * V + i] + acc[k][i];
+        for (int i = 0; i < V; ++i) {
+          const int c = ccol[k] + i;
+          if (i >= skip[k]) comb[c] = (gi == 0) ? acc[k][i] : comb[c] + acc[k][i];
+        }
       }
       if constexpr (X8) {
         if (own_x) {
@@ -1818,13 +1846,17 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_kernel(const Bwd
     }
     __syncthreads();
   }
+  if constexpr (ANY) {
+    for (int q = threadIdx.x; q < a.dim; q += blockDim.x) prow[q] = comb[q];
+    return;
+  }
   for (int q = threadIdx.x; q < a.dim / 4; q += blockDim.x)
     store16<VELOGRAD_DTYPE_F32>(prow, 4 * (int64_t)q, *reinterpret_cast<const u32x4*>(comb + 4 * q));
 }
 
 // ------------------------------------------------------------------------------------------
-// Backward, rows of any length and alignment that bwd_ring_kernel cannot take (odd lengths,
-// streams that start anywhere in a 16-byte line), in bwd_ring_kernel's walk and ring
+// Backward, short rows of any length and alignment (and longer ones where dx is grad_h itself), in
+// bwd_ring_kernel's walk and ring
 // (launch_plan.h: plan_bwd_ring_elem).  Element-strided lanes: lane lt of a row group holds
 // columns lt, lt + tpr, ..., lt + (M - 1) tpr, so each element load or store of a wave moves
 // one contiguous run of 64 elements; a column past the row's end loads the row's last element
@@ -2562,9 +2594,10 @@ RowPlan plan_fwd(int64_t dim, int elem_bytes, bool aligned, bool one_stream, boo
 }
 
 // `aligned8`: every stream starts on an 8-byte boundary (the weight on a 16-byte one), the
-// condition of the ring's kRing8 rows.
-BwdPlan plan_bwd(int64_t rows, int64_t dim, int elem_bytes, bool aligned, bool aligned8, int cus,
-                 bool rope, int64_t rope_seq) {
+// condition of the ring's kRing8 rows; `aligned_elem`: on their own elements' (kRingAny).
+BwdPlan plan_bwd(int64_t rows, int64_t dim, int elem_bytes, bool aligned, bool aligned8,
+                 bool aligned_elem, bool has_gh, bool dx_is_gh, int cus, bool rope,
+                 int64_t rope_seq) {
   const Tuning& t = tuning();
   if (!rope && t.bwd_ring) {
     const BwdPlan r = vg_plan::plan_bwd_ring(rows, dim, elem_bytes, aligned, cus, t.bwd_nv,
@@ -2585,8 +2618,19 @@ BwdPlan plan_bwd(int64_t rows, int64_t dim, int elem_bytes, bool aligned, bool a
                                   t.bwd_waves_per_cu);
   const BwdPlan p = vg_plan::plan_bwd(rows, dim, elem_bytes, aligned, cus, t.bwd_nv, t.bwd_block,
                                       t.bwd_waves_per_cu);
-  // rows the chunked kernels cannot take: the element-strided ring where it fits
+  // Rows the chunked kernels cannot take: short ones in the element-strided ring, the others in
+  // chunks from any element (unless dx is grad_h itself, see kRingAny), else element-strided as far
+  // as that goes.  Measured on MI355X, 16384 rows, elements (generic past 4096) / chunks, us: bf16 99
+  // 11.8 / 13.7, 200 11.6 / 11.5, 301 18.3 / 14.8, 1001 29.6 / 23.6, 2047 48.8 / 40.1, 2050 69.1 /
+  // 43.4, 3002 75.0 / 56.4, 4095 90.8 / 83.5, 8192 x 4099 68.2 / 49.5, 8192 x 8191 119 / 89; with
+  // grad_h 1001 36.2 / 29.1, 3002 99.5 / 71.1, 4095 119.5 / 111.4; fp32 401 20.8 / 21.7 but with
+  // grad_h 25.2 / 23.3, 1025 45.9 / 39.9, 2047 76.0 / 72.7.
   if (!p.rp.vec && t.bwd_ring) {
+    const bool short_row = dim <= (elem_bytes == 4 && !has_gh ? 512 : 192);
+    if (!short_row && aligned_elem && !dx_is_gh) {
+      const BwdPlan a = vg_plan::plan_bwd_ring_any(rows, dim, elem_bytes, cus);
+      if (a.ring) return a;
+    }
     const BwdPlan e = vg_plan::plan_bwd_ring_elem(rows, dim, elem_bytes, cus);
     if (e.elem_m > 0) return e;
   }
@@ -2716,6 +2760,15 @@ void launch_bwd_ring(const BwdArgs& a, const BwdPlan& b, hipStream_t st) {
                            st, a);
       return;
     }
+  }
+  if (b.any) {
+    if (b.rp.nv == 1)
+      hipLaunchKernelGGL((bwd_ring_kernel<DT, WDT, 1, F | kRingAny>), grid, block, b.lds_bytes, st,
+                         a);
+    else
+      hipLaunchKernelGGL((bwd_ring_kernel<DT, WDT, 2, F | kRingAny>), grid, block, b.lds_bytes, st,
+                         a);
+    return;
   }
   // rows of fewer chunks than the row group's lanes take the idle-lane variant
   if ((int64_t)b.rp.nv * b.rp.tpr * Codec<DT>::kVec != a.dim) {
@@ -3118,8 +3171,15 @@ int32_t run_bwd(const void* grad_y, const void* saved, int32_t saved_is_h, const
                         (!grad_h || (aligned8p(grad_h) && ld_ok8(ld_grad_h, eb))) &&
                         (!weight || aligned16(weight));
   const bool rope = rope_seq > 0;
-  BwdPlan plan = plan_bwd(rows, dim, eb, aligned, aligned8, cus, rope, rope_seq);
-  const int64_t plan_dim = plan.x8 ? dim - 4 : dim;  // the columns the row plan lays out
+  const bool aligned_elem = elem_ok_ptr(grad_y, eb) && elem_ok_ptr(saved, eb) &&
+                            elem_ok_ptr(dx, eb) && elem_ok_ptr(dres, eb) &&
+                            elem_ok_ptr(grad_h, eb) && elem_ok_ptr(weight, elem_bytes_of(w_dtype));
+  BwdPlan plan = plan_bwd(rows, dim, eb, aligned, aligned8, aligned_elem, grad_h != nullptr,
+                          dx == grad_h, cus, rope, rope_seq);
+  // the columns the row plan lays out
+  const int64_t plan_dim = plan.x8    ? dim - 4
+                           : plan.any ? (dim + 16 / eb - 1) / (16 / eb) * (16 / eb)
+                                      : dim;
   // bwd_vec_kernel's RoPE walk keeps its step rotations (two floats per pair: dim floats) in the
   // same dynamic LDS as the group combine, one after the other.
   if (rope && plan.rp.vec && !plan.ring && !plan.rope_direct)
@@ -3130,8 +3190,10 @@ int32_t run_bwd(const void* grad_y, const void* saved, int32_t saved_is_h, const
       plan.rp.block <= vg_plan::kRingBlock && (int64_t)plan.elem_m * plan.rp.tpr >= dim;
   if ((plan.elem_m > 0 ? !elem_ok : !vg_plan::row_plan_valid(plan.rp, plan_dim, eb)) ||
       plan.wgs < 1 || plan.wgs > INT32_MAX || plan.lds_bytes > 64 * 1024 ||
-      (plan.ring && !rope && (!vg_plan::ring_eligible(plan.rp, plan_dim, eb) ||
-                              plan.rp.block > vg_plan::kRingBlock)) ||
+      (plan.ring && !rope &&
+       ((plan.any ? dim < 16 / eb || plan.rp.nv > vg_plan::kRingMaxNV
+                  : !vg_plan::ring_eligible(plan.rp, plan_dim, eb)) ||
+        plan.rp.block > vg_plan::kRingBlock)) ||
       (plan.x8 && (rope || !plan.ring || eb != 2 || dim % 8 != 4 || plan.rp.nv != 1 ||
                    !aligned8)) ||
       (plan.ring && rope && (!vg_plan::rope_ring_eligible(plan.rp, dim, eb) ||
@@ -3145,9 +3207,14 @@ int32_t run_bwd(const void* grad_y, const void* saved, int32_t saved_is_h, const
 
   float* partial = nullptr;
   if (dweight != nullptr) {
-    const size_t need = (size_t)plan.wgs * (size_t)dim * sizeof(float);
+    size_t need = (size_t)plan.wgs * (size_t)dim * sizeof(float);
     if (static_scratch) {
-      // velograd_rmsnorm_residual_bwd_noalloc: the partial rows go to the library's own array
+      // velograd_rmsnorm_residual_bwd_noalloc: the partial rows go to the library's own array.
+      // Wide rows that the chunked kernels cannot take are held to the generic kernel's need.
+      if (plan.any && dim > vg_plan::kRingElemMaxM * vg_plan::kRingBlock)
+        need = (size_t)vg_plan::plan_bwd(rows, dim, eb, false, cus, tuning().bwd_nv,
+                                         tuning().bwd_block, tuning().bwd_waves_per_cu).wgs *
+               (size_t)dim * sizeof(float);
       if (need > kNoAllocScratchBytes)
         return fail(VELOGRAD_ERR_WORKSPACE_TOO_SMALL,
                     "bwd_noalloc: dweight needs %zu bytes of scratch for rows=%lld dim=%lld, above "
