@@ -2520,38 +2520,46 @@ __global__ __launch_bounds__(kGenericBlock) void bwd_generic_kernel(const BwdArg
 // ------------------------------------------------------------------------------------------
 // dweight stage 2: dweight[j] = sum over partial rows p = 0..nparts-1, in a fixed order.
 // A workgroup owns 64 columns; wave w sums rows p = w, w + W, ... and the W wave sums are
-// added in wave order.
+// added in wave order.  The kernel is bound by the round trips to the partial rows that another
+// XCD wrote, not by their bytes, so a wave's rows are read in batches of 16 loads in flight (four
+// for at most 64 partial rows), the last batch filled up with the last row (read, not added): one
+// round trip up to 256 partial rows.  A loop over the rows past the last whole batch waited for
+// each, up to 15 times with under 256 partial rows (short tensors, several row groups a
+// workgroup).  The whole backward, such a loop / batches (bf16, graph replays, us): 512 x 768 7.8 /
+// 6.0, 512 x 1024 8.7 / 6.8, 128 x 4096 9.4 / 7.6, 200 x 4096 10.7 / 8.1, 512 x 4096 9.3 / 9.0.
 // ------------------------------------------------------------------------------------------
 constexpr int kReduceBlock = 1024;
 __global__ __launch_bounds__(kReduceBlock) void dweight_reduce_kernel(const float* partial,
                                                                        int32_t nparts,
                                                                        int32_t dim,
                                                                        float* dweight) {
-  __shared__ float red[kReduceBlock / kWave][kWave];
+  constexpr int kWaves = kReduceBlock / kWave;
+  __shared__ float red[kWaves][kWave];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
-  const int nw = blockDim.x / kWave;
   const int col = blockIdx.x * kWave + lane;
   float s = 0.0f;
-  if (col < dim) {
-    // Batches of 16 loads in flight per lane (one HBM round trip for the usual 256 partial rows
-    // over 16 waves); the additions keep ascending p order.
-    constexpr int kBatch = 16;
-    int p = wave;
-    for (; p + (kBatch - 1) * nw < nparts; p += kBatch * nw) {
+  auto sum_rows = [&](auto batch) {
+    constexpr int kBatch = decltype(batch)::value;
+    for (int p = wave; p < nparts; p += kBatch * kWaves) {
       float v[kBatch];
 #pragma unroll
-      for (int b = 0; b < kBatch; ++b) v[b] = partial[(int64_t)(p + b * nw) * dim + col];
+      for (int b = 0; b < kBatch; ++b)
+        v[b] = partial[(int64_t)min(p + b * kWaves, nparts - 1) * dim + col];
 #pragma unroll
-      for (int b = 0; b < kBatch; ++b) s += v[b];
+      for (int b = 0; b < kBatch; ++b) s = p + b * kWaves < nparts ? s + v[b] : s;
     }
-    for (; p < nparts; p += nw) s += partial[(int64_t)p * dim + col];
+  };
+  if (col < dim) {
+    if (nparts <= 4 * kWaves) sum_rows(std::integral_constant<int, 4>{});
+    else sum_rows(std::integral_constant<int, 16>{});
   }
   red[wave][lane] = s;
   __syncthreads();
   if (wave == 0 && col < dim) {
     float t = red[0][lane];
-    for (int w = 1; w < nw; ++w) t += red[w][lane];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) t += red[w][lane];
     dweight[col] = t;
   }
 }
