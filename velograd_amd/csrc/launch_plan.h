@@ -522,6 +522,28 @@ inline BwdPlan plan_bwd_rope_ring(int64_t rows, int64_t dim, int elem_bytes, boo
   return b;
 }
 
+// The same over rows that the chunked layout does not fit or fills only in part (even lengths from
+// one chunk up, any alignment; bwd_rope_ring_kernel's ANY, the last chunk overlapping the one
+// before it).
+inline BwdPlan plan_bwd_rope_ring_any(int64_t rows, int64_t dim, int elem_bytes, int cus) {
+  BwdPlan b;
+  b.rp = RowPlan{false, 0, kGenericBlock, 1, kGenericBlock};
+  b.wgs = 0;
+  b.lds_bytes = 0;
+  if ((elem_bytes != 2 && elem_bytes != 4) || dim < 16 / elem_bytes || dim % 2 != 0) return b;
+  const int V = 16 / elem_bytes;
+  const int64_t chunks = (dim + V - 1) / V;
+  const int nv = chunks <= kRingBlock ? 1 : 2;
+  const int64_t tpr = (chunks + (int64_t)nv * kWave - 1) / ((int64_t)nv * kWave) * kWave;
+  if (tpr > kRingBlock) return b;
+  // the plan of the whole row group, its combine over the row's own columns
+  b = plan_bwd_rope_ring(rows, tpr * nv * V, elem_bytes, true, cus);
+  if (!b.ring) return b;
+  if (b.rp.groups > 1) b.lds_bytes -= (size_t)(tpr * nv * V - dim) * sizeof(float);
+  b.any = true;
+  return b;
+}
+
 // Whether `slots` row slots walking `rows` rows (slot s: rows s, s + slots, ...) see positions
 // (row % seq) that only advance by `slots` or return to the walk's first one: slots is a
 // multiple or a divisor of seq, or no walk reaches the end of a sequence.
@@ -644,6 +666,8 @@ inline size_t bwd_workspace_bytes(int64_t rows, int64_t dim, int cus, int prefer
       if (rg.ring && rg.wgs > most) most = rg.wgs;
       const BwdPlan rr = plan_bwd_rope_ring(rows, dim, sizes[si], al != 0, cus);
       if (rr.ring && rr.wgs > most) most = rr.wgs;
+      const BwdPlan rra = plan_bwd_rope_ring_any(rows, dim, sizes[si], cus);
+      if (rra.ring && rra.wgs > most) most = rra.wgs;
       const BwdPlan r8 = plan_bwd_ring8(rows, dim, sizes[si], cus, ring_block, ring_wgs_per_cu);
       if (r8.ring && r8.wgs > most) most = r8.wgs;
       const BwdPlan re = plan_bwd_ring_elem(rows, dim, sizes[si], cus);

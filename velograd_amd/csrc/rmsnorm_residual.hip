@@ -267,6 +267,8 @@ struct BwdArgs {
   int32_t iters;  // rows visited per slot = ceil(rows / slots)
   int64_t rope_seq;            // kRopeG: positions per outer index (row position = row % rope_seq)
   float rope_c_hi, rope_c_lo;  // kRopeG: log2(base) / half as an unevaluated float sum
+  double rope_ratio;           // kRopeG: base^(-2/dim), one pair's frequency over the one before
+  bool rope_back;              // the ring: a walk past a sequence's end returns to its first position
 };
 
 // Output modes of the forward kernels.
@@ -281,44 +283,13 @@ constexpr int kOutDtypeLateH = 5;  // as kOutDtype, with h stored after the row 
 // row at position pos turns by pos * freq_i, freq_i = base^(-2i/dim) = 2^-(i * c) with
 // c = log2(base) / half.  c arrives as c_hi + c_lo (from double on the host); freq_i and the
 // angle pos * freq_i are formed in double, as the reference's Python floats are, and the angle is
-// reduced exactly to [-1/2, 1/2] revolutions before a float32 sincospi, so cos and sin are within
+// reduced exactly to [-1/2, 1/2] revolutions before a float32 cos and sin, so they are within
 // a few float32 ulps at any position (a float32 angle would carry pos * freq_i * 2^-24 radians of
 // error: 0.016 rad at position 2.6e5).
 constexpr double kInv2PiD = 0.159154943091895335768883763372514362;
 constexpr double kTwoPiD = 6.283185307179586476925286766559005768;
 __device__ __forceinline__ double rope_freq(int i, float c_hi, float c_lo) {
   return exp2(-(double)i * ((double)c_hi + (double)c_lo));
-}
-
-// cos and sin of pair i's angle at position pos.
-__device__ __forceinline__ void rope_cos_sin(int64_t pos, int i, float c_hi, float c_lo, float& c,
-                                             float& s) {
-  const double rev = (double)pos * rope_freq(i, c_hi, c_lo) * kInv2PiD;
-  sincospif(2.0f * (float)(rev - rint(rev)), &s, &c);
-}
-
-// The frequencies of a thread's pairs in a strided loop (pairs i0, i0 + stride, ...): the first
-// from exp2, each next one the previous times base^(-2 stride / dim), in double (a few double
-// ulps over a row, far below the float32 rotation's rounding), so the generic kernels pay one
-// double exp2 per row and thread instead of one per pair.
-struct RopeFreqWalk {
-  double f, ratio;
-  __device__ RopeFreqWalk(int i0, int stride, float c_hi, float c_lo) {
-    const double c = (double)c_hi + (double)c_lo;
-    f = exp2(-(double)i0 * c);
-    ratio = exp2(-(double)stride * c);
-  }
-  __device__ double next() {
-    const double v = f;
-    f *= ratio;
-    return v;
-  }
-};
-
-// cos and sin at position pos of the pair whose frequency is fr (as rope_cos_sin)
-__device__ __forceinline__ void rope_cos_sin_f(int64_t pos, double fr, float& c, float& s) {
-  const double rev = (double)pos * fr * kInv2PiD;
-  sincospif(2.0f * (float)(rev - rint(rev)), &s, &c);
 }
 
 // A double angle in revolutions reduced exactly to [-1/2, 1/2], and the cos and sin of such an
@@ -349,6 +320,35 @@ __device__ __forceinline__ void cos_sin_turn(float rev, float& c, float& s) {
                                     ((uint32_t)(q & 2) << 30));
   c = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, odd ? s0 : c0) ^
                                     ((uint32_t)((q + 1) & 2) << 30));
+}
+
+// cos and sin of pair i's angle at position pos.
+__device__ __forceinline__ void rope_cos_sin(int64_t pos, int i, float c_hi, float c_lo, float& c,
+                                             float& s) {
+  cos_sin_turn(rope_frac((double)pos * rope_freq(i, c_hi, c_lo) * kInv2PiD), c, s);
+}
+
+// The frequencies of a thread's pairs in a strided loop (pairs i0, i0 + stride, ...): the first
+// from exp2, each next one the previous times base^(-2 stride / dim), in double (a few double
+// ulps over a row, far below the float32 rotation's rounding), so the generic kernels pay one
+// double exp2 per row and thread instead of one per pair.
+struct RopeFreqWalk {
+  double f, ratio;
+  __device__ RopeFreqWalk(int i0, int stride, float c_hi, float c_lo) {
+    const double c = (double)c_hi + (double)c_lo;
+    f = exp2(-(double)i0 * c);
+    ratio = exp2(-(double)stride * c);
+  }
+  __device__ double next() {
+    const double v = f;
+    f *= ratio;
+    return v;
+  }
+};
+
+// cos and sin at position pos of the pair whose frequency is fr (as rope_cos_sin)
+__device__ __forceinline__ void rope_cos_sin_f(int64_t pos, double fr, float& c, float& s) {
+  cos_sin_turn(rope_frac((double)pos * fr * kInv2PiD), c, s);
 }
 
 // cos and sin of |x| <= 1 in double by their Taylor series through x^14 and x^13 (truncation below
@@ -2031,7 +2031,7 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_elem_kernel(cons
 // (two workgroups of fewer than 512 threads fit a CU); two chunks per thread, one workgroup per
 // CU, within 256.
 // ------------------------------------------------------------------------------------------
-template <int DT, int WDT, int NV>
+template <int DT, int WDT, int NV, bool ANY>
 __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope_ring_kernel(
     const BwdArgs a) {
   using C = Codec<DT>;
@@ -2072,45 +2072,59 @@ __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope
   // 1 / dim is exact for a power of two, so s * (1 / dim) has the bits of s / dim
   const bool dim_pow2 = (a.dim & (a.dim - 1)) == 0;
   const float inv_dim = 1.0f / (float)a.dim;
-  auto col_of = [&](int k) { return (int64_t)(lt + k * tpr) * V; };
-  // pair e's frequency: base^(-2i/dim), i its pair index in the row
-  auto freq_of = [&](int e) {
+  // first column of the lane's chunk k; the columns not its own to sum, and whether it has any
+  auto col_of = [&](int k) { return ANY ? min((lt + k * tpr) * V, a.dim - V) : (lt + k * tpr) * V; };
+  auto skip_of = [&](int k) { return ANY ? (lt + k * tpr) * V - col_of(k) : 0; };
+  auto own = [&](int k) { return !ANY || skip_of(k) < V; };
+  auto load_chunk = [&](const void* base, int64_t e) {
+    if constexpr (ANY) return load16_any_stream<DT>(base, e);
+    else return load16_stream<DT>(base, e);
+  };
+  // pair e's turns a position: base^(-2i/dim) / (2 pi), i its pair index in the row
+  auto turns_of = [&](int e) {
     if constexpr (kTablesInLds) return freq_lds[e * bd + tid];
-    else return rope_freq((lt + (e / P) * tpr) * P + e % P, a.rope_c_hi, a.rope_c_lo);
+    else
+      return rope_freq(col_of(e / P) / 2 + e % P, a.rope_c_hi, a.rope_c_lo) * kInv2PiD;
   };
 
   float wf[NV][V], acc[NV][V];
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     WeightChunk<DT, WDT> wc;
-    wc.load(a.w, col_of(k));
+    if constexpr (ANY) {
+      if (a.w != nullptr) wc.load_any(a.w, col_of(k));
+    } else {
+      wc.load(a.w, col_of(k));
+    }
     wc.unpack(a.w != nullptr, wf[k]);
 #pragma unroll
     for (int i = 0; i < V; ++i) acc[k][i] = 0.0f;
   }
-  // one pair at a time (a double sincos holds many registers; the walk needs them)
+  // one pair at a time (the walk needs the registers): its turns a position, the first of a chunk
+  // from exp2, each next one by the double ratio; the rotation through S positions in double
+  double g = 0.0;
 #pragma unroll 1
   for (int e = 0; e < NP; ++e) {
-    const double f = rope_freq((lt + (e / P) * tpr) * P + e % P, a.rope_c_hi, a.rope_c_lo);
+    g = e % P == 0 ? rope_freq(col_of(e / P) / 2, a.rope_c_hi, a.rope_c_lo) * kInv2PiD
+                   : g * a.rope_ratio;
+    const double rev = (double)S * g;
     double sv, cv;
-    sincos((double)S * f, &sv, &cv);
+    cos_sin_turn_d(rev - rint(rev), cv, sv);
     step_lds[e * bd + tid] = float2{(float)cv, (float)sv};
     if constexpr (kTablesInLds) {
-      freq_lds[e * bd + tid] = f;
-      // the rotation at the walk's first position: double angle, reduced exactly, float sincospi
-      const double rev = (double)pos0 * f * kInv2PiD;
+      freq_lds[e * bd + tid] = g;
+      // the rotation at the walk's first position: double angle, reduced exactly, float cos and sin
       float s0, c0;
-      sincospif(2.0f * (float)(rev - rint(rev)), &s0, &c0);
+      cos_sin_turn(rope_frac((double)pos0 * g), c0, s0);
       first_lds[e * bd + tid] = float2{c0, s0};
     }
   }
   float cr[NP], sr[NP];
-  // the rotations at position p evaluated afresh: double angle, exact reduction, float sincospi
+  // the rotations at position p evaluated afresh: double angle, exact reduction, float cos and sin
   auto evaluate_at = [&](int64_t p) {
 #pragma unroll
     for (int e = 0; e < NP; ++e) {
-      const double rev = (double)p * freq_of(e) * kInv2PiD;
-      sincospif(2.0f * (float)(rev - rint(rev)), &sr[e], &cr[e]);
+      cos_sin_turn(rope_frac((double)p * turns_of(e)), cr[e], sr[e]);
     }
   };
   auto restore_first = [&]() {
@@ -2137,8 +2151,8 @@ __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope
     r = a.inv_rms[rw];
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-      gv[k] = load16_stream<DT>(a.g, rw * a.ld_g + col_of(k));
-      hv[k] = load16_stream<DT>(a.saved, rw * a.ld_s + col_of(k));
+      gv[k] = load_chunk(a.g, rw * a.ld_g + col_of(k));
+      hv[k] = load_chunk(a.saved, rw * a.ld_s + col_of(k));
     }
   };
   // The backward of one row (bwd_vec_kernel's with kSavedIsH | kRopeG); `ok` = the row exists.
@@ -2160,7 +2174,10 @@ __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope
 #pragma unroll
       for (int i = 0; i < V; ++i) xh[k][i] = xh[k][i] * r;
 #pragma unroll
-      for (int i = 0; i < V; ++i) s = __builtin_fmaf(gf[k][i] * wf[k][i], xh[k][i], s);
+      for (int i = 0; i < V; ++i) {
+        const float t = __builtin_fmaf(gf[k][i] * wf[k][i], xh[k][i], s);
+        s = ANY && i < skip_of(k) ? s : t;
+      }
     }
     s = row_sum(s, tpr, grp, red[it & 1]);
     const float m = dim_pow2 ? s * inv_dim : s / (float)a.dim;
@@ -2169,7 +2186,10 @@ __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope
       float d[V];
 #pragma unroll
       for (int i = 0; i < V; ++i) d[i] = r * __builtin_fmaf(-xh[k][i], m, gf[k][i] * wf[k][i]);
-      if (ok) store16_stream<DT>(a.dx, row * a.ld_dx + col_of(k), C::pack(d));
+      if (ok && own(k)) {
+        if constexpr (ANY) store16_any_stream<DT>(a.dx, row * a.ld_dx + col_of(k), C::pack(d));
+        else store16_stream<DT>(a.dx, row * a.ld_dx + col_of(k), C::pack(d));
+      }
 #pragma unroll
       for (int i = 0; i < V; ++i) {
         acc[k][i] = ok ? __builtin_fmaf(gf[k][i], xh[k][i], acc[k][i]) : acc[k][i];
@@ -2183,9 +2203,14 @@ __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope
     pos += S;
     ++since;
     if (pos >= seq) {
-      pos = pos0;
       since = 0;
-      restore_first();
+      if (a.rope_back) {
+        pos = pos0;
+        restore_first();
+      } else {
+        pos = (row + S) % seq;
+        evaluate_at(pos);
+      }
     } else if (since == kRopeAnchorRows) {
       since = 0;
       evaluate_at(pos);
@@ -2232,6 +2257,12 @@ __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope
   if (groups == 1) {
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
+      if constexpr (ANY) {
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+          if (i >= skip_of(k)) prow[col_of(k) + i] = acc[k][i];
+        continue;
+      }
 #pragma unroll
       for (int q = 0; q < V / 4; ++q)
         store16<VELOGRAD_DTYPE_F32>(prow, col_of(k) + 4 * q,
@@ -2244,11 +2275,17 @@ __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope
 #pragma unroll
       for (int k = 0; k < NV; ++k) {
 #pragma unroll
-        for (int i = 0; i < V; ++i)
-          comb[col_of(k) + i] = (gi == 0) ? acc[k][i] : comb[col_of(k) + i] + acc[k][i];
+        for (int i = 0; i < V; ++i) {
+          const int c = col_of(k) + i;
+          if (i >= skip_of(k)) comb[c] = (gi == 0) ? acc[k][i] : comb[c] + acc[k][i];
+        }
       }
     }
     __syncthreads();
+  }
+  if constexpr (ANY) {
+    for (int q = threadIdx.x; q < a.dim; q += blockDim.x) prow[q] = comb[q];
+    return;
   }
   for (int q = threadIdx.x; q < a.dim / 4; q += blockDim.x)
     store16<VELOGRAD_DTYPE_F32>(prow, 4 * (int64_t)q, *reinterpret_cast<const u32x4*>(comb + 4 * q));
@@ -2607,6 +2644,7 @@ BwdPlan plan_bwd(int64_t rows, int64_t dim, int elem_bytes, bool aligned, bool a
                  bool aligned_elem, bool has_gh, bool dx_is_gh, int cus, bool rope,
                  int64_t rope_seq) {
   const Tuning& t = tuning();
+  (void)rope_seq;
   if (!rope && t.bwd_ring) {
     const BwdPlan r = vg_plan::plan_bwd_ring(rows, dim, elem_bytes, aligned, cus, t.bwd_nv,
                                              t.ring_block, t.ring_wgs_per_cu);
@@ -2619,7 +2657,9 @@ BwdPlan plan_bwd(int64_t rows, int64_t dim, int elem_bytes, bool aligned, bool a
   }
   if (rope && t.bwd_ring) {
     const BwdPlan r = vg_plan::plan_bwd_rope_ring(rows, dim, elem_bytes, aligned, cus);
-    if (r.ring && vg_plan::rope_walk_ok(rows, r.wgs * r.rp.groups, rope_seq)) return r;
+    if (r.ring) return r;
+    const BwdPlan ra = vg_plan::plan_bwd_rope_ring_any(rows, dim, elem_bytes, cus);
+    if (ra.ring && aligned_elem) return ra;
   }
   if (rope)
     return vg_plan::plan_bwd_rope(rows, dim, elem_bytes, aligned, cus, t.bwd_nv, t.bwd_block,
@@ -2834,10 +2874,20 @@ void launch_bwd_flags(const BwdArgs& a, const BwdPlan& b, hipStream_t st) {
   }
   if constexpr ((F & kRopeG) != 0) {
     if (b.ring) {
-      if (p.nv == 2)
-        hipLaunchKernelGGL((bwd_rope_ring_kernel<DT, WDT, 2>), grid, block, lds, st, a);
-      else
-        hipLaunchKernelGGL((bwd_rope_ring_kernel<DT, WDT, 1>), grid, block, lds, st, a);
+      switch (p.nv * 2 + (b.any ? 1 : 0)) {
+        case 2:
+          hipLaunchKernelGGL((bwd_rope_ring_kernel<DT, WDT, 1, false>), grid, block, lds, st, a);
+          break;
+        case 3:
+          hipLaunchKernelGGL((bwd_rope_ring_kernel<DT, WDT, 1, true>), grid, block, lds, st, a);
+          break;
+        case 4:
+          hipLaunchKernelGGL((bwd_rope_ring_kernel<DT, WDT, 2, false>), grid, block, lds, st, a);
+          break;
+        default:
+          hipLaunchKernelGGL((bwd_rope_ring_kernel<DT, WDT, 2, true>), grid, block, lds, st, a);
+          break;
+      }
       return;
     }
     if (b.rope_direct) {
@@ -3198,14 +3248,14 @@ int32_t run_bwd(const void* grad_y, const void* saved, int32_t saved_is_h, const
       plan.rp.block <= vg_plan::kRingBlock && (int64_t)plan.elem_m * plan.rp.tpr >= dim;
   if ((plan.elem_m > 0 ? !elem_ok : !vg_plan::row_plan_valid(plan.rp, plan_dim, eb)) ||
       plan.wgs < 1 || plan.wgs > INT32_MAX || plan.lds_bytes > 64 * 1024 ||
+      (plan.ring && plan.any && (dim < 16 / eb || plan.rp.block > vg_plan::kRingBlock)) ||
       (plan.ring && !rope &&
        ((plan.any ? dim < 16 / eb || plan.rp.nv > vg_plan::kRingMaxNV
                   : !vg_plan::ring_eligible(plan.rp, plan_dim, eb)) ||
         plan.rp.block > vg_plan::kRingBlock)) ||
       (plan.x8 && (rope || !plan.ring || eb != 2 || dim % 8 != 4 || plan.rp.nv != 1 ||
                    !aligned8)) ||
-      (plan.ring && rope && (!vg_plan::rope_ring_eligible(plan.rp, dim, eb) ||
-                             !vg_plan::rope_walk_ok(rows, plan.wgs * plan.rp.groups, rope_seq))) ||
+      (plan.ring && rope && !plan.any && !vg_plan::rope_ring_eligible(plan.rp, dim, eb)) ||
       (rope && plan.rp.vec && !plan.ring && !plan.rope_direct &&
        plan.rp.block > vg_plan::max_block_for_nv_rope(plan.rp.nv)) ||
       (plan.rope_direct && (!rope || plan.rp.block > vg_plan::max_block_for_nv(plan.rp.nv))))
@@ -3268,6 +3318,8 @@ int32_t run_bwd(const void* grad_y, const void* saved, int32_t saved_is_h, const
   const double c = rope ? log2((double)rope_base) / (double)(dim / 2) : 0.0;
   a.rope_c_hi = (float)c;
   a.rope_c_lo = (float)(c - (double)a.rope_c_hi);
+  a.rope_ratio = exp2(-c);
+  a.rope_back = rope && vg_plan::rope_walk_ok(rows, slots, rope_seq);
   VG_DISPATCH_TYPES(dtype, w_dtype, (launch_bwd<kD, kW>(a, saved_is_h != 0, rope, plan, st)));
   int32_t rc = check_launch(rope ? "velograd_rmsnorm_rope_bwd" : "velograd_rmsnorm_residual_bwd");
   if (rc != 0 || dweight == nullptr) return rc;
