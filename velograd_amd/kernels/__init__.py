@@ -206,6 +206,10 @@ def _forward_fast(x: torch.Tensor, residual: Optional[torch.Tensor],
     return y, h, inv_rms
 
 
+def _tensors_or_none(*ts: Any) -> bool:
+    return all(t is None or isinstance(t, torch.Tensor) for t in ts)
+
+
 def _check_min_mean_sq(min_mean_sq: float) -> float:
     min_mean_sq = float(min_mean_sq)
     if not (math.isfinite(min_mean_sq) and min_mean_sq >= 0.0):
@@ -223,6 +227,13 @@ def _forward_device(x: torch.Tensor, residual: Optional[torch.Tensor],
         fast = _forward_fast(x, residual, weight, eps, min_mean_sq)
         if fast is not None:
             return fast
+    elif _tensors_or_none(residual, weight):
+        fp = _lib.fastpath()
+        if fp is not None:
+            fmt = -1 if mx is None else (_lib.MX_E4M3 if mx == "e4m3" else _lib.MX_E2M1)
+            out = fp.forward_quantised(x, residual, weight, float(eps), fmt)
+            if out:
+                return out[0], out[1], (x if residual is None else out[2]), out[3]
     lib = _lib.load()
     device = x.device
     code = _dtype_code(x, "x")
@@ -315,6 +326,12 @@ def _backward_device(grad_out: torch.Tensor, saved: torch.Tensor,
                      weight: Optional[torch.Tensor], inv_rms: torch.Tensor,
                      saved_is_h: bool, dresidual_out: Optional[torch.Tensor],
                      grad_h: Optional[torch.Tensor] = None):
+    fp = _lib.fastpath()
+    if (fp is not None and isinstance(saved, torch.Tensor) and isinstance(inv_rms, torch.Tensor)
+            and _tensors_or_none(weight, dresidual_out, grad_h)):
+        out = fp.backward(grad_out, saved, weight, inv_rms, bool(saved_is_h), dresidual_out, grad_h)
+        if out:
+            return out[0], out[1]
     lib = _lib.load()
     device = grad_out.device
     code = _dtype_code(grad_out, "grad_out")
@@ -538,6 +555,12 @@ def _rope_device(t: torch.Tensor, layout, h_dim: int, theta: float, inverse: boo
 
 def _rope(q: Any, k: Optional[Any], head_dim: Optional[int], theta: float, inverse: bool):
     on_device = _is_device_tensor(q)
+    if on_device and _tensors_or_none(k) and (head_dim is None or isinstance(head_dim, int)):
+        fp = _lib.fastpath()
+        if fp is not None:
+            out = fp.rope(q, k, int(head_dim or 0), float(theta), inverse)
+            if out:
+                return out[0], out[1]
     if not on_device:
         device = _require_gpu()
         q_np = np.asarray(q.detach().cpu().numpy() if isinstance(q, torch.Tensor) else q,
@@ -608,6 +631,11 @@ def fused_rope_interleaved(x: torch.Tensor, base: float = 10000.0,
         raise TypeError("fused_rope_interleaved takes torch tensors on a ROCm device")
     if x.dim() < 2:
         raise ValueError("fused_rope_interleaved: x must be [..., seq, dim]")
+    fp = _lib.fastpath()
+    if fp is not None:
+        out = fp.rope_interleaved(x, float(base), bool(inverse))
+        if out:
+            return out[0]
     seq, dim = x.shape[-2], x.shape[-1]
     if dim % 2 != 0:
         raise ValueError(f"fused_rope_interleaved: dim={dim} must be even (RoPE pairs)")
@@ -677,6 +705,11 @@ def rmsnorm_rope_forward(x: torch.Tensor, weight: Optional[torch.Tensor] = None,
     if x.dim() < 2:
         raise ValueError("rmsnorm_rope_forward: x must be [..., seq, dim]")
     min_mean_sq = _check_min_mean_sq(min_mean_sq)
+    fp = _lib.fastpath()
+    if fp is not None and _tensors_or_none(residual, weight):
+        out = fp.norm_rope(x, residual, weight, float(eps), float(base), min_mean_sq)
+        if out:
+            return out[0], (x if residual is None else out[1]), out[2]
     seq, d = x.shape[-2], x.shape[-1]
     if d % 2 != 0:
         raise ValueError(f"rmsnorm_rope_forward: dim={d} must be even (RoPE pairs)")
@@ -722,6 +755,12 @@ def rmsnorm_rope_backward(grad_y: torch.Tensor, h: torch.Tensor,
         raise TypeError("rmsnorm_rope_backward takes torch tensors on a ROCm device")
     if grad_y.dim() < 2:
         raise ValueError("rmsnorm_rope_backward: grad_y must be [..., seq, dim]")
+    fp = _lib.fastpath()
+    if (fp is not None and isinstance(h, torch.Tensor) and isinstance(inv_rms, torch.Tensor)
+            and _tensors_or_none(weight)):
+        out = fp.norm_rope_backward(grad_y, h, weight, inv_rms, float(base))
+        if out:
+            return out[0], out[1]
     seq, d = grad_y.shape[-2], grad_y.shape[-1]
     if d % 2 != 0:
         raise ValueError(f"rmsnorm_rope_backward: dim={d} must be even (RoPE pairs)")
