@@ -165,11 +165,14 @@ VG_HOST_DEVICE inline uint32_t xcd_item(uint32_t b, uint32_t n, int run_log2) {
 // keep an XCD's requests on neighbouring pages and let the lines that two ragged rows share meet
 // in one L2.  The forward is bound by HBM; measured (bf16, alternating processes, best of 3 to 6;
 // rows by block index / runs of 8, 16, 32 and 64 workgroups, us): 16384 x 4096 86.1 / 86.0, 86.8,
-// 84.1, 89.5; 16384 x 8192 172.1 / 170.3, 169.5, 168.7, 168.8; 8192 x 16384 177.1 / 173.4, 171.8,
-// 173.4, 179.9; 32768 x 2048 86.7 / 88.8, 86.6, 88.4, 84.3; 32768 x 768 35.0 / 34.1, 34.0, 33.6,
-// 33.6; 16384 x 4095 (generic kernel) 100.6 / 97.8, 97.3, 95.8, 94.8; fp32 8192 x 4096 87.5 /
-// 87.9, 86.6, 85.6, 84.7.  Without a residual 16384 x 4096 ran 43.7 against 44.3, quantised to
-// fp8 75.5 against 75.8.  256 KiB is the best or within 2% of it in each.
+// 84.1, 89.5; 16384 x 8192 172.1 / 170.3, 169.5, 168.7, 168.8; 32768 x 2048 86.7 / 88.8, 86.6,
+// 88.4, 84.3; 32768 x 768 35.0 / 34.1, 34.0, 33.6, 33.6; 16384 x 4095 (generic kernel) 100.6 /
+// 97.8, 97.3, 95.8, 94.8; fp32 8192 x 4096 87.5 / 87.9, 86.6, 85.6, 84.7.  256 KiB is the best or
+// within 2% of it in each.  Two chunks a thread (one process, the same buffers in turn; by block
+// index / runs of 128, 256 and 512 KiB): 8192 x 16384 176.7 / 174.5, 174.1, 175.8; fp8 16384 x 4096
+// 76.2 / 76.1, 75.7, 76.8, 4096 x 4096 22.8 / 22.5, 22.5, 22.8, 32768 x 1024 39.5 / 39.4, 39.2,
+// 40.1; MXFP8 16384 x 4096 77.6 / 77.5, 76.5, 78.7; MXFP4 16384 x 4096 71.8 / 71.3, 71.0, 71.4;
+// without a residual 16384 x 4096 44.9 / 44.8, 44.9, 45.9.
 constexpr int64_t kXcdRunBytes = 256 << 10;
 constexpr int kXcdRunMaxLog2 = 6;
 inline int xcd_run_log2(int64_t row_bytes, int groups) {

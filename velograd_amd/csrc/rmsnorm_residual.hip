@@ -477,21 +477,28 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
   u32x4 xv[NV], rv[NV];
   WeightChunk<DT, WDT> wc[NV];
   // ANY: the lane's element outside the chunks
+  constexpr bool kAllStray = ROWS == kRowsAnyNoRes && (MX || OUT == kOutFp8Row);
   const bool own_s = ANY && row_ok && lt < a.dim - nchunk * V;
   const int j_s = lt < head ? lt : lt + nchunk * V;
   typename C::Raw x_raw{}, r_raw{};
   typename Codec<WDT>::Raw w_raw{};
+  // No wait may fall between these loads (16384 x 4095 bf16 100.9 us with one, 94.2 without; two
+  // chunks a thread: MXFP4 32768 x 1024 39.4 / 36.8, without a residual 16384 x 4096 48.6 / 45.1),
+  // so they stand under no per-lane condition, which would merge each value with the one that the
+  // other lanes keep: a lane without a chunk reads the row's last columns, a row past the end the
+  // last row.
+  const int64_t rw = row_ok ? row : a.rows - 1;
   if constexpr (ANY) {
-    // No wait may fall between these loads (16384 x 4095 bf16 100.9 us with one, 94.2 without), so
-    // the raw elements come first and are decoded at the row sum, what is absent is
-    // read from x instead, a lane without a chunk reads the row's last columns and a row past
-    // the end reads the last row.
-    if (own_s) {
-      x_raw = static_cast<const typename C::Raw*>(a.x)[row * a.ld_x + j_s];
-      if (has_res) r_raw = static_cast<const typename C::Raw*>(a.res)[row * a.ld_res + j_s];
-      w_raw = static_cast<const typename Codec<WDT>::Raw*>(has_w ? a.w : a.x)[has_w ? j_s : 0];
+    // The raw elements come first and are decoded at the row sum; what is absent is read from x.
+    // Quantised outputs without a residual, short of loads, take them on every lane for the same
+    // reason (16384 x 255 fp8 9.6 / 9.3 us); the others ran up to 2% slower that way (more
+    // requests).
+    if (kAllStray || own_s) {
+      const int j = own_s ? j_s : 0;
+      x_raw = static_cast<const typename C::Raw*>(a.x)[rw * a.ld_x + j];
+      if (has_res) r_raw = static_cast<const typename C::Raw*>(a.res)[rw * a.ld_res + j];
+      w_raw = static_cast<const typename Codec<WDT>::Raw*>(has_w ? a.w : a.x)[has_w ? j : 0];
     }
-    const int64_t rw = row_ok ? row : a.rows - 1;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       const int col = min(col_of(lt + k * tpr), a.dim - V);
@@ -500,20 +507,23 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
       if (has_w) wc[k].load_any(a.w, col);
     }
   } else {
+    int col[NV];
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-      const int c = lt + k * tpr;
-      xv[k] = u32x4{0u, 0u, 0u, 0u};
-      rv[k] = u32x4{0u, 0u, 0u, 0u};
-      if (row_ok && c < nchunk) {
-        xv[k] = load_chunk(a.x, row * a.ld_x + (int64_t)c * V);
-        if (has_res) rv[k] = load_chunk(a.res, row * a.ld_res + (int64_t)c * V);
-      }
+      col[k] = min(lt + k * tpr, nchunk - 1) * V;
+      xv[k] = load_chunk(a.x, rw * a.ld_x + col[k]);
+      if (has_res) rv[k] = load_chunk(a.res, rw * a.ld_res + col[k]);
     }
+    if (has_w) {
+#pragma unroll
+      for (int k = 0; k < NV; ++k) wc[k].load(a.w, col[k]);
+    }
+    // one wait for all of them, before the first store of h: a wait after that, at the next
+    // chunk's first use, would be for the store as well
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-      const int c = lt + k * tpr;
-      wc[k].load((has_w && c < nchunk) ? a.w : nullptr, (int64_t)c * V);
+      forget(xv[k]);
+      forget(rv[k]);
     }
   }
 
@@ -541,8 +551,10 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
       for (int i = 0; i < V; ++i) p += hf[i] * hf[i];
       ss += c < nchunk ? p : 0.0f;
     } else {
+      float t = ss;
 #pragma unroll
-      for (int i = 0; i < V; ++i) ss += hf[i] * hf[i];
+      for (int i = 0; i < V; ++i) t += hf[i] * hf[i];
+      ss = c < nchunk ? t : ss;
     }
     if (!kLateH && write_h && row_ok && c < nchunk)
       store_chunk(a.h, row * a.ld_h + col_of(c), C::pack(hf));
@@ -554,7 +566,7 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
     h_s = C::decode1(x_raw);
     if (has_res) h_s = h_s + C::decode1(r_raw);
     if (has_w) w_s = Codec<WDT>::decode1(w_raw);
-    ss += h_s * h_s;
+    ss += own_s ? h_s * h_s : 0.0f;
     if (write_h && own_s) C::store1(a.h, row * a.ld_h + j_s, h_s);
   }
   ss = row_sum(ss, tpr, grp, red);
