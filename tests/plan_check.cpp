@@ -416,6 +416,12 @@ int main() {
     const RowPlan f4s = plan_rows(8192, 4, true, 4, kFwdOrder);
     CHECK(f4s.vec && f4s.nv == 4 && f4s.tpr == 512, "fwd nv 4 at fp32 8192");
   }
+  // Forward rows of any length with a residual: two chunks a thread in up to two waves, else one.
+  for (int64_t dim : {1001, 2047, 2055, 2056, 2201, 3002, 3076, 4095}) {
+    const RowPlan p = plan_any_rows(dim, 2, false);
+    CHECK(p.vec && p.nv == (dim < 2056 ? 2 : 1), "any-row forward at %lld: nv %d", (long long)dim,
+          p.nv);
+  }
   // The allocation-free backward refuses fp32 2048 x 16384 (tests/test_zz_no_alloc.py): on 256
   // CUs with the default tuning, every plan the backward can pick for that shape (aligned or
   // not, with or without the ring) needs more partial rows than its 16 MiB scratch holds, while

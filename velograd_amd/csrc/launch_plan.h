@@ -124,11 +124,13 @@ inline RowPlan plan_rows(int64_t dim, int elem_bytes, bool aligned, int prefer_n
 // streams that start anywhere): fwd_vec_kernel's any-alignment form takes them from one chunk up,
 // laid out over the dim / V whole chunks a row can hold.  Two chunks a thread where a row has
 // enough for that without a residual or with a quantised output (the orders above), else up to
-// kAnyTwoChunks chunks; longer rows one chunk a thread up to the workgroup bound.  Measured with a
-// residual (bf16, 16384 rows; one chunk and h stored early / two chunks and h stored late, us):
-// 1001 26.8 / 25.3, 1535 40.0 / 38.7, 2047 51.6 / 50.0, 3002 71.9 / 70.3, but 4095 95.6 / 98.4 and
-// fp32 8192 x 4099 90.0 / 93.2.
-constexpr int kAnyTwoChunks = 384;
+// kAnyTwoChunks chunks (two waves); longer rows one chunk a thread up to the workgroup bound.
+// Measured with a residual (bf16, 16384 rows; one chunk and h stored early / two chunks and h stored
+// late, us): 1001 26.8 / 25.3, 1535 40.0 / 38.7, 2047 51.6 / 50.0, but in three waves, alone in their
+// workgroup, 2201 51.1 / 54.5, 2562 58.6 / 62.7, 3002 66.3 / 70.6, 3076 69.7 / 74.7 (rows of
+// 8n + 4 elements in 8-byte halves 72.0), 4095 95.6 / 98.4, fp32 1281 58.6 / 62.1, 1537 72.6 / 76.8,
+// 8192 x 4099 90.0 / 93.2.
+constexpr int kAnyTwoChunks = 256;
 inline RowPlan plan_any_rows(int64_t dim, int elem_bytes, bool two_first) {
   RowPlan p{false, 0, kGenericBlock, 1, kGenericBlock};
   if (elem_bytes != 2 && elem_bytes != 4) return p;
