@@ -418,10 +418,15 @@ int main() {
   }
   // Forward rows of any length with a residual: two chunks a thread in up to two waves, else one.
   for (int64_t dim : {1001, 2047, 2055, 2056, 2201, 3002, 3076, 4095}) {
-    const RowPlan p = plan_any_rows(dim, 2, false);
+    const RowPlan p = plan_any_rows(dim, 2, true, false);
     CHECK(p.vec && p.nv == (dim < 2056 ? 2 : 1), "any-row forward at %lld: nv %d", (long long)dim,
           p.nv);
   }
+  // Without one, plain rows of more than 896 chunks keep the generic kernel.
+  CHECK(plan_any_rows(7175, 2, false, false).vec && !plan_any_rows(7176, 2, false, false).vec &&
+            !plan_any_rows(4095, 4, false, false).vec && !plan_any_rows(14001, 2, false, false).vec &&
+            plan_any_rows(14001, 2, true, false).vec && plan_any_rows(14001, 2, false, true).vec,
+        "any-row forward without a residual");
   // The allocation-free backward refuses fp32 2048 x 16384 (tests/test_zz_no_alloc.py): on 256
   // CUs with the default tuning, every plan the backward can pick for that shape (aligned or
   // not, with or without the ring) needs more partial rows than its 16 MiB scratch holds, while

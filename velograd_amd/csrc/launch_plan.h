@@ -131,13 +131,21 @@ inline RowPlan plan_rows(int64_t dim, int elem_bytes, bool aligned, int prefer_n
 // 8n + 4 elements in 8-byte halves 72.0), 4095 95.6 / 98.4, fp32 1281 58.6 / 62.1, 1537 72.6 / 76.8,
 // 8192 x 4099 90.0 / 93.2.
 constexpr int kAnyTwoChunks = 256;
-inline RowPlan plan_any_rows(int64_t dim, int elem_bytes, bool two_first) {
+// Without a residual and with y in the activation dtype, rows of more chunks than this keep the
+// generic kernel, whose 256-thread workgroups leave a CU more rows to overlap than one row group of
+// eight to sixteen waves.  Measured (8192 rows; generic kernel / any-row form, us): bf16 4099 32.0 /
+// 27.3, 6149 41.9 / 39.9, 7001 46.0 / 45.8, 7503 48.3 / 50.4, 8191 50.2 / 53.0, 10003 63.3 / 70.5,
+// 14001 89.1 / 100.7; fp32 3501 41.0 / 41.1, 4095 47.5 / 48.3, 5001 57.7 / 61.5, 8191 95.1 / 98.2.
+constexpr int kAnyOneStreamChunks = 896;
+// `residual`: the forward adds one; `quantised`: y is stored as fp8 or MX codes.
+inline RowPlan plan_any_rows(int64_t dim, int elem_bytes, bool residual, bool quantised) {
   RowPlan p{false, 0, kGenericBlock, 1, kGenericBlock};
   if (elem_bytes != 2 && elem_bytes != 4) return p;
   const int V = 16 / elem_bytes;
   if (dim < V) return p;
   const int64_t chunks = dim / V;
-  const bool two = chunks > kWave && (two_first || chunks <= kAnyTwoChunks);
+  if (!residual && !quantised && chunks > kAnyOneStreamChunks) return p;
+  const bool two = chunks > kWave && (!residual || quantised || chunks <= kAnyTwoChunks);
   const int nv = two || chunks > max_block_for_nv(1) ? 2 : 1;
   const int64_t tpr = (chunks + (int64_t)kWave * nv - 1) / ((int64_t)kWave * nv) * kWave;
   if (tpr > max_block_for_nv(nv)) return p;

@@ -1020,9 +1020,9 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void fwd_elem_kernel(const Fwd
 }
 
 // ------------------------------------------------------------------------------------------
-// Forward, the rows that the kernels above do not take (longer than their registers hold, shorter
-// than a chunk with a quantised output, the RoPE output on rows that are not whole chunks, streams
-// off their element's alignment): one row per workgroup, two passes over the row (the second
+// Forward, the rows that the kernels above do not take (longer than their registers hold, wide any
+// rows without a residual (plan_any_rows), rows shorter than a chunk with a quantised or RoPE
+// output, streams off their element's alignment): one row per workgroup, two passes over the row (the second
 // re-reads x and residual, normally from L2, and recomputes the identical fp32 h).
 // ------------------------------------------------------------------------------------------
 template <int DT, int WDT, int OUT>
@@ -3096,7 +3096,7 @@ int32_t run_fwd(const char* what, int out, const void* x, const void* residual,
     elem_m = vg_plan::elem_per_lane(dim);
     if (elem_m > 0) p = vg_plan::plan_elem_rows(dim);
   } else if (!p.vec && out != kOutRopeI && aligned_elem) {
-    const RowPlan pa = vg_plan::plan_any_rows(dim, eb, residual == nullptr || out != kOutDtype);
+    const RowPlan pa = vg_plan::plan_any_rows(dim, eb, residual != nullptr, out != kOutDtype);
     if (pa.vec) {
       p = pa;
       any = true;
