@@ -36,6 +36,10 @@ int main() {
     }
   }
   if (xcd_run_log2(8192, 1) != 5) return printf("8 KiB rows\n"), 1;
+  // wide rows of the generic kernel keep their block's index, narrower ones go in runs
+  if (xcd_run_log2(22010, 1, true) != 0 || xcd_run_log2(65536, 1, true) != 0 ||
+      xcd_run_log2(18002, 1, true) != xcd_run_log2(18002, 1))
+    return printf("generic rows\n"), 1;
   printf("xcd_run_check ok\n");
   return 0;
 }

@@ -185,7 +185,13 @@ VG_HOST_DEVICE inline uint32_t xcd_item(uint32_t b, uint32_t n, int run_log2) {
 // without a residual 16384 x 4096 44.9 / 44.8, 44.9, 45.9.
 constexpr int64_t kXcdRunBytes = 256 << 10;
 constexpr int kXcdRunMaxLog2 = 6;
-inline int xcd_run_log2(int64_t row_bytes, int groups) {
+// Rows of more than kXcdGenericRowBytes in the generic kernel, which reads them twice, go by block
+// index: 4096 rows, by block index / in runs, us: bf16 without a residual 9001 (twice the rows) 58.6
+// / 57.7, 11005 37.8 / 38.5, 14001 45.3 / 47.3, 32768 103.8 / 106.9, with one 20000 135.6 / 139.0,
+// 32768 231.0 / 234.5; fp32 5001 (twice) 58.9 / 57.9, 16384 108.6 / 112.3; MXFP8 20000 2621 / 2710.
+constexpr int64_t kXcdGenericRowBytes = 20 << 10;
+inline int xcd_run_log2(int64_t row_bytes, int groups, bool generic = false) {
+  if (generic && row_bytes > kXcdGenericRowBytes) return 0;
   const int64_t wg = row_bytes * groups > 0 ? row_bytes * groups : 1;
   int n = 0;
   while (n < kXcdRunMaxLog2 && (wg << (n + 1)) * 3 <= kXcdRunBytes * 4) ++n;

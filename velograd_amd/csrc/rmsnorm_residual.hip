@@ -3130,7 +3130,7 @@ int32_t run_fwd(const char* what, int out, const void* x, const void* residual,
   a.ms_floor = ms_floor;
   a.rope_seq = rope_seq > 0 ? rope_seq : 1;
   a.rope_half = (int32_t)(dim / 2);
-  a.run_log2 = vg_plan::xcd_run_log2(dim * eb, p.groups);
+  a.run_log2 = vg_plan::xcd_run_log2(dim * eb, p.groups, !p.vec && elem_m == 0);
   const double c = (rope_theta > 0.0f && dim >= 2) ? log2((double)rope_theta) / (double)(dim / 2)
                                                    : 0.0;
   a.rope_c_hi = (float)c;
