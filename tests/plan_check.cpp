@@ -427,6 +427,13 @@ int main() {
             !plan_any_rows(4095, 4, false, false).vec && !plan_any_rows(14001, 2, false, false).vec &&
             plan_any_rows(14001, 2, true, false).vec && plan_any_rows(14001, 2, false, true).vec,
         "any-row forward without a residual");
+  // Backward rows of any length: 2-byte ones of one wave of chunks go element by element, those
+  // past 256 elements on short tensors only.
+  CHECK(bwd_elem_first(1 << 20, 256, 2, true, 256) && !bwd_elem_first(16384, 257, 2, false, 256) &&
+            bwd_elem_first(8191, 257, 2, false, 256) && bwd_elem_first(64, 512, 2, true, 256) &&
+            !bwd_elem_first(64, 513, 2, false, 256) && !bwd_elem_first(8192, 511, 2, false, 256) &&
+            bwd_elem_first(64, 512, 4, false, 256) && !bwd_elem_first(64, 193, 4, true, 256),
+        "element-first backward");
   // The allocation-free backward refuses fp32 2048 x 16384 (tests/test_zz_no_alloc.py): on 256
   // CUs with the default tuning, every plan the backward can pick for that shape (aligned or
   // not, with or without the ring) needs more partial rows than its 16 MiB scratch holds, while

@@ -469,6 +469,19 @@ inline RowPlan plan_elem_rows(int64_t dim) {
   return p;
 }
 
+// Whether a backward over rows that the chunked layout does not fit goes element by element rather
+// than in chunks from any element (plan_bwd_ring_any).  2-byte rows of up to 512 elements are one
+// wave of chunks, eight row groups a workgroup, whose combine alone costs a short tensor more than
+// the chunks save; up to 256 elements both have eight.  Measured (bf16; elements / chunks, us): 193
+// at 128 rows 7.2 / 8.0, 16384 13.4 / 14.2, 49152 24.3 / 24.6; 257 at 64 rows 6.5 / 8.1, 2048 8.5 /
+// 10.0, 4096 10.4 / 10.3, 16384 18.0 / 14.4; 511 at 128 rows 7.0 / 8.4, 3072 10.3 / 11.4, 6144 12.6 /
+// 13.0, 8192 13.6 / 13.7, 10240 15.3 / 14.1; 513 at 64 rows 7.7 / 7.0.
+constexpr int kAnyOneWaveRowsPerCu = 32;
+inline bool bwd_elem_first(int64_t rows, int64_t dim, int elem_bytes, bool has_gh, int cus) {
+  if (elem_bytes == 4) return dim <= (has_gh ? 192 : 512);
+  return dim <= 256 || (dim <= 512 && rows < (int64_t)kAnyOneWaveRowsPerCu * cus);
+}
+
 // The element-strided ring backward: plan_elem_rows' row groups, one workgroup per CU.
 inline BwdPlan plan_bwd_ring_elem(int64_t rows, int64_t dim, int elem_bytes, int cus) {
   BwdPlan b;

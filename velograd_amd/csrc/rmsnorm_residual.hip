@@ -2678,16 +2678,16 @@ BwdPlan plan_bwd(int64_t rows, int64_t dim, int elem_bytes, bool aligned, bool a
                                   t.bwd_waves_per_cu);
   const BwdPlan p = vg_plan::plan_bwd(rows, dim, elem_bytes, aligned, cus, t.bwd_nv, t.bwd_block,
                                       t.bwd_waves_per_cu);
-  // Rows the chunked kernels cannot take: short ones in the element-strided ring, the others in
-  // chunks from any element (unless dx is grad_h itself, see kRingAny), else element-strided as far
-  // as that goes.  Measured on MI355X, 16384 rows, elements (generic past 4096) / chunks, us: bf16 99
-  // 11.8 / 13.7, 200 11.6 / 11.5, 301 18.3 / 14.8, 1001 29.6 / 23.6, 2047 48.8 / 40.1, 2050 69.1 /
+  // Rows the chunked kernels cannot take: short ones (bwd_elem_first) in the element-strided ring,
+  // the others in chunks from any element (unless dx is grad_h itself, see kRingAny), else
+  // element-strided as far as that goes.  Measured on MI355X, 16384 rows, elements (generic past
+  // 4096) / chunks, us: bf16 99 11.8 / 13.7, 301 18.3 / 14.8, 1001 29.6 / 23.6, 2047 48.8 / 40.1, 2050 69.1 /
   // 43.4, 3002 75.0 / 56.4, 4095 90.8 / 83.5, 8192 x 4099 68.2 / 49.5, 8192 x 8191 119 / 89; with
   // grad_h 1001 36.2 / 29.1, 3002 99.5 / 71.1, 4095 119.5 / 111.4; fp32 401 20.8 / 21.7 but with
   // grad_h 25.2 / 23.3, 1025 45.9 / 39.9, 2047 76.0 / 72.7.
   if (!p.rp.vec && t.bwd_ring) {
-    const bool short_row = dim <= (elem_bytes == 4 && !has_gh ? 512 : 192);
-    if (!short_row && aligned_elem && !dx_is_gh) {
+    if (!vg_plan::bwd_elem_first(rows, dim, elem_bytes, has_gh, cus) && aligned_elem &&
+        !dx_is_gh) {
       const BwdPlan a = vg_plan::plan_bwd_ring_any(rows, dim, elem_bytes, cus);
       if (a.ring) return a;
     }
