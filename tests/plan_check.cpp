@@ -434,6 +434,56 @@ int main() {
             !bwd_elem_first(64, 513, 2, false, 256) && !bwd_elem_first(8192, 511, 2, false, 256) &&
             bwd_elem_first(64, 512, 4, false, 256) && !bwd_elem_first(64, 193, 4, true, 256),
         "element-first backward");
+  // The norm + RoPE forward's tiles: every row in exactly one, at its position, by workgroups and
+  // row groups that fit; sequences shorter than a tile still fill it.
+  long tiles = 0;
+  for (int64_t seq : {1, 2, 3, 4, 5, 7, 64, 1023, 4097}) {
+    for (int64_t outer : {1, 2, 3, 5, 300, 1025, 2051}) {
+      if (seq * outer > 300000) continue;
+      for (int64_t dim : {2, 8, 10, 512, 768, 1000, 4100, 8192, 8194, 16384, 16386}) {
+        for (int eb = 2; eb <= 4; eb += 2) {
+          for (int res = 0; res < 2; ++res) {
+            const int64_t rows = seq * outer;
+            const RopeTilePlan t = plan_rope_tiles(rows, dim, eb, seq, res != 0);
+            const int V = 16 / eb;
+            CHECK(t.rp.vec == (dim >= V && (dim + V - 1) / V <= 2048), "rope tiles at %lld x %d",
+                  (long long)dim, eb);
+            if (!t.rp.vec) continue;
+            CHECK((int64_t)t.rp.nv * t.rp.tpr * V >= dim && t.rp.tpr % kWave == 0 &&
+                      t.rp.block == t.rp.tpr * t.rp.groups && t.rp.nv >= 1 && t.rp.nv <= 2 &&
+                      t.rp.block <= max_block_for_nv(t.rp.nv) &&
+                      (t.tile == 1 || t.tile == 2 || t.tile == 4) &&
+                      t.tile <= rope_tile_most(eb, t.rp.nv, res != 0),
+                  "rope tile plan %lld x %d", (long long)dim, eb);
+            std::vector<char> seen(rows, 0);
+            for (int64_t i = 0; i < t.wgs * t.rp.groups; ++i) {
+              const RopeTile q = rope_tile((uint32_t)i, (uint32_t)rows, (uint32_t)seq, t.tile,
+                                           t.across);
+              CHECK(q.n >= 1 && q.n <= t.tile, "rope tile of %d rows", q.n);
+              for (int u = 0; u < q.n; ++u) {
+                const int64_t row = (int64_t)q.first + (int64_t)u * q.step;
+                CHECK(row < rows && row % seq == q.pos + (t.across ? 0 : u),
+                      "rope tile row %lld of %lld x %lld", (long long)row, (long long)outer,
+                      (long long)seq);
+                if (q.ok && row < rows) ++seen[row];
+              }
+            }
+            ++tiles;
+            bool once = true;
+            for (char c : seen) once = once && c == 1;
+            CHECK(once, "rope tiles of %lld x %lld x %lld", (long long)outer, (long long)seq,
+                  (long long)dim);
+          }
+        }
+      }
+    }
+  }
+  CHECK(plan_rope_tiles(16384, 4096, 2, 1, false).tile == 4 &&
+            plan_rope_tiles(16384, 4096, 2, 2, false).tile == 4 &&
+            plan_rope_tiles(16384, 4096, 2, 1, true).tile == 2 &&
+            plan_rope_tiles(16384, 4096, 4, 3, false).tile == 4,
+        "whole tiles over short sequences");
+  printf("rope tile plans checked: %ld\n", tiles);
   // The allocation-free backward refuses fp32 2048 x 16384 (tests/test_zz_no_alloc.py): on 256
   // CUs with the default tuning, every plan the backward can pick for that shape (aligned or
   // not, with or without the ring) needs more partial rows than its 16 MiB scratch holds, while

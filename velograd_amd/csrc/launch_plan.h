@@ -632,21 +632,32 @@ inline BwdPlan plan_bwd_rope(int64_t rows, int64_t dim, int elem_bytes, bool ali
 
 // Tiles of the norm + RoPE forward (fwd_rope_tile_kernel): row groups of one chunk a thread up to
 // the workgroup bound (the row's last chunk may overlap the one before it), else of two; tiles of
-// four consecutive positions, two with a residual (its loads double the registers: 16384 x 4096
-// bf16 88.2 us against 91.6, 8192 x 16384 195 against 259), halved while they are longer than the
-// sequence or leave fewer than kRopeTileMinWgs workgroups (bf16 dim 4096, tiles of 1 / 2 / 4, us: 64
-// rows 3.5 / 3.9 / 4.5, 512 4.8 / 4.4 / 5.0, 2048 11.7 / 8.8 / 8.1).  `rp.vec` false: a row shorter
-// than a chunk or longer than the registers hold.
+// up to rope_tile_most rows, halved while they leave fewer than kRopeTileMinWgs workgroups (bf16 dim
+// 4096, tiles of 1 / 2 / 4, us: 64 rows 3.5 / 3.9 / 4.5, 512 4.8 / 4.4 / 5.0, 2048 11.7 / 8.8 / 8.1) or
+// are longer than what they cut.  A tile's rows are consecutive positions of one sequence, or, of
+// sequences shorter than a tile (decode steps), one position of consecutive sequences, so that its
+// rotations still serve all of its rows (bf16, cut to the sequence / across sequences, us: 16384 x
+// 4096 in sequences of 1 72.5 / 46.2, of 2 54.2 / 48.1, of 3 62.0 / 46.6, 65536 x 768 of 1 70.4 /
+// 34.8).  `rp.vec` false: a row shorter than a chunk or longer than the registers hold.
+//
+// With a residual its loads double the registers, and two chunks a thread or fp32's double rotations
+// do so again: tiles of 1 / 2 / 4 there, us: bf16 16384 x 4096 - / 88.2 / 91.6, 8192 x 16384 188 / 205 /
+// 259, 4096 x 12288 70.9 / 76.5; fp32 8192 x 2048 44.8 / 45.8, 8192 x 4096 90.8 / 93.1, 4096 x 8192
+// 90.2 / 94.9, 16384 x 1024 45.5 / 45.1.
+constexpr int rope_tile_most(int elem_bytes, int nv, bool residual) {
+  return !residual ? 4 : elem_bytes == 4 || nv == 2 ? 1 : 2;
+}
 struct RopeTilePlan {
   RowPlan rp;
-  int tile;     // positions a tile
+  int tile;     // rows a tile
+  bool across;  // of consecutive sequences, at one position
   int64_t wgs;  // workgroups, rp.groups tiles each
 };
 constexpr int64_t kRopeTileMinWgs = 256;
 
 inline RopeTilePlan plan_rope_tiles(int64_t rows, int64_t dim, int elem_bytes, int64_t seq,
                                     bool residual) {
-  RopeTilePlan t{RowPlan{false, 0, kGenericBlock, 1, kGenericBlock}, 1, 0};
+  RopeTilePlan t{RowPlan{false, 0, kGenericBlock, 1, kGenericBlock}, 1, false, 0};
   if ((elem_bytes != 2 && elem_bytes != 4) || rows < 1 || seq < 1) return t;
   const int V = 16 / elem_bytes;
   if (dim < V) return t;
@@ -660,10 +671,39 @@ inline RopeTilePlan plan_rope_tiles(int64_t rows, int64_t dim, int elem_bytes, i
   p.tpr = (int)tpr;
   p.groups = p.tpr >= 256 ? 1 : 256 / p.tpr;
   p.block = p.tpr * p.groups;
-  auto wgs = [&](int r) { return (rows / seq * ((seq + r - 1) / r) + p.groups - 1) / p.groups; };
-  t.tile = residual ? 2 : 4;
-  while (t.tile > 1 && (t.tile > seq || wgs(t.tile) < kRopeTileMinWgs)) t.tile /= 2;
+  t.tile = rope_tile_most(elem_bytes, nv, residual);
+  t.across = seq < t.tile;
+  const int64_t cut = t.across ? rows / seq : seq;  // what the tiles cut, rows / cut times
+  auto wgs = [&](int r) { return (rows / cut * ((cut + r - 1) / r) + p.groups - 1) / p.groups; };
+  while (t.tile > 1 && (t.tile > cut || wgs(t.tile) < kRopeTileMinWgs)) t.tile /= 2;
   t.wgs = wgs(t.tile);
+  return t;
+}
+
+// The rows of tile i, r of them at most: first, first + step, ..., n of them, the first at position
+// pos and the others at the next ones or (`across`) at the same.  Tiles past the last one give the
+// last (ok false).
+struct RopeTile {
+  uint32_t first, step, pos;
+  int n;
+  bool ok;
+};
+VG_HOST_DEVICE inline RopeTile rope_tile(uint32_t i, uint32_t rows, uint32_t seq, int r,
+                                         bool across) {
+  const uint32_t outer = rows / seq;
+  const uint32_t cut = across ? outer : seq, other = across ? seq : outer;
+  const uint32_t per = (cut + r - 1) / r;
+  RopeTile t;
+  t.ok = i < per * other;
+  if (!t.ok) i = per * other - 1;
+  // consecutive tiles hold neighbouring rows: across, the positions of the same sequences
+  const uint32_t q = i / (across ? other : per);
+  const uint32_t m = i - q * (across ? other : per);
+  const uint32_t at = (across ? q : m) * r;  // in what is cut
+  t.pos = across ? m : at;
+  t.first = across ? at * seq + m : q * seq + at;
+  t.step = across ? seq : 1;
+  t.n = (int)(cut - at < (uint32_t)r ? cut - at : (uint32_t)r);
   return t;
 }
 

@@ -249,6 +249,8 @@ struct FwdArgs {
   float rope_c_hi, rope_c_lo;  // kOutRopeI: log2(base) / half as an unevaluated float sum
   double rope_log2_step, rope_ratio;  // kOutRopeI: -log2(base) / half and 2 to it
   bool rope_small_step;       // kOutRopeI: base >= 1, so a position's step is 1 radian at most
+  bool rope_across;           // kOutRopeI: a tile is one position of consecutive sequences
+  double rope_step_rad;       // kOutRopeI: 2 pi, or 0 across sequences
 };
 
 struct BwdArgs {
@@ -708,15 +710,16 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
 }
 
 // ------------------------------------------------------------------------------------------
-// Forward with the model's RoPE on y (kOutRopeI): a one-shot grid of tiles.  A row group takes R
-// consecutive positions of one sequence (a position past the sequence's end re-reads the last one
-// and stores nothing): all their loads are in flight at once, the rotations are formed while they
+// Forward with the model's RoPE on y (kOutRopeI): a one-shot grid of tiles.  A row group takes the R
+// rows of a tile (launch_plan.h: rope_tile): consecutive positions of one sequence, or one position
+// of consecutive short sequences (a row past the end re-reads the last one and stores nothing): all
+// their loads are in flight at once, the rotations are formed while they
 // are, one barrier serves the R row sums, and consecutive tiles run on one XCD (xcd_item).
 // Angles, as the reference's Python floats form them (functional.py:302-305): pair j turns
 // g_j = base^(-2j/dim) / (2 pi) revolutions per position, in double (one exp2 per chunk, its next
 // pairs by the double ratio); the tile's first position times g_j in double is reduced exactly to
 // [-1/2, 1/2] revolutions before a float cos and sin (cos_sin_turn), and the next positions
-// advance that by the step rotation, at most R - 1 times: in float for bf16/fp16 outputs (3
+// advance that by the step rotation (none across sequences), at most R - 1 times: in float for bf16/fp16 outputs (3
 // float32 ulps a step at most, far below their rounding), in double for fp32 ones.
 // Short tiles cost trigonometry, which the vector units pay (28 instructions an element at four
 // positions), long ones parallelism; a walk of 16 or 32 strided rows per workgroup instead, its
@@ -740,20 +743,18 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_rope_tile_kernel(con
   __shared__ float red[kMaxWavesPerRow][4 * RQ];
 
   const int tpr = a.tpr;
-  const int grp = threadIdx.x / tpr;
+  // a row group is whole waves: its tile and rows are wave-uniform, and so scalar
+  const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x / (uint32_t)tpr);
   const int lt = threadIdx.x - grp * tpr;
   const int groups = blockDim.x / tpr;
-  // the tile: positions s0 .. s0 + ns - 1 of sequence o
-  const uint32_t seq = (uint32_t)a.rope_seq;
-  const uint32_t tps = (seq + R - 1) / R;
-  const uint32_t tiles = (uint32_t)(a.rows / seq) * tps;
-  const uint32_t item = xcd_item(blockIdx.x, gridDim.x, a.run_log2) * groups + grp;
-  const bool ok = item < tiles;
-  const uint32_t tile = ok ? item : tiles - 1;
-  const uint32_t o = tile / tps;
-  const uint32_t s0 = (tile - o * tps) * R;
-  const int ns = (int)min(seq - s0, (uint32_t)R);
-  const int64_t row0 = (int64_t)o * seq + s0;
+  // the tile: ns rows, step apart, the first at position s0
+  const vg_plan::RopeTile tile =
+      vg_plan::rope_tile(xcd_item(blockIdx.x, gridDim.x, a.run_log2) * groups + grp,
+                         (uint32_t)a.rows, (uint32_t)a.rope_seq, R, a.rope_across);
+  const bool ok = tile.ok;
+  const uint32_t s0 = tile.pos;
+  const int ns = tile.n;
+  const int64_t row0 = tile.first, step = tile.step;
   const bool has_w = a.w != nullptr;
   const int nchunk = ANY ? (a.dim + V - 1) / V : a.dim / V;
   int col[NV];    // first column of the lane's chunks
@@ -769,7 +770,7 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_rope_tile_kernel(con
   WeightChunk<DT, WDT> wc[NV];
 #pragma unroll
   for (int u = 0; u < R; ++u) {
-    const int64_t row = row0 + (u < ns ? u : ns - 1);
+    const int64_t row = row0 + (u < ns ? u : ns - 1) * step;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       if constexpr (ANY) {
@@ -803,12 +804,14 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_rope_tile_kernel(con
       cr[e] = c0;
       sr[e] = s0f;
       if constexpr (R > 1) {
+        // (a step of 0, across sequences, gives 1 and 0 exactly)
+        const double turns = a.rope_small_step || !a.rope_across ? g : 0.0;
         if constexpr (DT == VELOGRAD_DTYPE_F32) {
-          if (a.rope_small_step) cos_sin_small_d(g * kTwoPiD, cs[e], sn[e]);
-          else cos_sin_turn_d(g - rint(g), cs[e], sn[e]);
+          if (a.rope_small_step) cos_sin_small_d(g * a.rope_step_rad, cs[e], sn[e]);
+          else cos_sin_turn_d(turns - rint(turns), cs[e], sn[e]);
         } else {
-          if (a.rope_small_step) cos_sin_small((float)(g * kTwoPiD), cs[e], sn[e]);
-          else cos_sin_turn(rope_frac(g), cs[e], sn[e]);
+          if (a.rope_small_step) cos_sin_small((float)(g * a.rope_step_rad), cs[e], sn[e]);
+          else cos_sin_turn(rope_frac(turns), cs[e], sn[e]);
         }
       }
       g *= a.rope_ratio;
@@ -868,7 +871,8 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_rope_tile_kernel(con
       t += dpp_move<0x128>(t);
       const float mean = t / (float)a.dim;
       const float ir = 1.0f / __builtin_sqrtf(floor_mean_sq(mean, a.ms_floor) + a.eps);
-      if (lt < kWave && w == 0 && ok && u < ns && a.inv_rms != nullptr) a.inv_rms[row0 + u] = ir;
+      if (lt < kWave && w == 0 && ok && u < ns && a.inv_rms != nullptr)
+        a.inv_rms[row0 + u * step] = ir;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         if (4 * q + j < R)
@@ -884,7 +888,7 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_rope_tile_kernel(con
   for (int k = 0; k < NV; ++k) wc[k].unpack(has_w, wf[k]);
 #pragma unroll
   for (int u = 0; u < R; ++u) {
-    const int64_t row = row0 + u;
+    const int64_t row = row0 + u * step;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       float hf[V];
@@ -2769,16 +2773,20 @@ void launch_fwd_any(const FwdArgs& a, const RowPlan& p, hipStream_t st) {
 template <int DT, int WDT, int NV, bool RES, bool ANY>
 void launch_rope_tile(const FwdArgs& a, const vg_plan::RopeTilePlan& p, hipStream_t st) {
   const dim3 grid((uint32_t)p.wgs), block(p.rp.block);
-  if constexpr (!RES) {
+  constexpr int kMost = vg_plan::rope_tile_most(Codec<DT>::kBytes, NV, RES);
+  if constexpr (kMost >= 4) {
     if (p.tile == 4) {
       hipLaunchKernelGGL((fwd_rope_tile_kernel<DT, WDT, NV, RES, 4, ANY>), grid, block, 0, st, a);
       return;
     }
   }
-  if (p.tile == 2)
-    hipLaunchKernelGGL((fwd_rope_tile_kernel<DT, WDT, NV, RES, 2, ANY>), grid, block, 0, st, a);
-  else
-    hipLaunchKernelGGL((fwd_rope_tile_kernel<DT, WDT, NV, RES, 1, ANY>), grid, block, 0, st, a);
+  if constexpr (kMost >= 2) {
+    if (p.tile == 2) {
+      hipLaunchKernelGGL((fwd_rope_tile_kernel<DT, WDT, NV, RES, 2, ANY>), grid, block, 0, st, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((fwd_rope_tile_kernel<DT, WDT, NV, RES, 1, ANY>), grid, block, 0, st, a);
 }
 
 template <int DT, int WDT>
@@ -3138,12 +3146,16 @@ int32_t run_fwd(const char* what, int out, const void* x, const void* residual,
   a.rope_log2_step = -c;
   a.rope_ratio = exp2(-c);
   a.rope_small_step = rope_theta >= 1.0f;
+  a.rope_across = false;
+  a.rope_step_rad = kTwoPiD;
   hipStream_t st = static_cast<hipStream_t>(hip_stream);
   if (out == kOutRopeI && aligned_elem) {
     const vg_plan::RopeTilePlan t =
         vg_plan::plan_rope_tiles(rows, dim, eb, rope_seq, residual != nullptr);
     if (t.rp.vec) {
       a.tpr = t.rp.tpr;
+      a.rope_across = t.across;
+      if (t.across) a.rope_step_rad = 0.0;
       a.run_log2 = vg_plan::xcd_run_log2(dim * eb * t.tile, t.rp.groups);
       const bool any = !aligned || dim % (16 / eb) != 0;
       VG_DISPATCH_TYPES(dtype, w_dtype, (launch_rope_tiles<kD, kW>(a, t, any, st)));
