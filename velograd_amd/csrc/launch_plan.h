@@ -572,9 +572,19 @@ inline BwdPlan plan_bwd_rope_ring_any(int64_t rows, int64_t dim, int elem_bytes,
   b = plan_bwd_rope_ring(rows, tpr * nv * V, elem_bytes, true, cus);
   if (!b.ring) return b;
   if (b.rp.groups > 1) b.lds_bytes -= (size_t)(tpr * nv * V - dim) * sizeof(float);
+  // fp32's step rotations are double, in the place of the first rotations with one chunk a thread;
+  // with two, those or the 2-byte rows' frequencies come on top
+  if (nv == 2) b.lds_bytes += (size_t)b.rp.block * nv * (V / 2) * sizeof(double);
   b.any = true;
   return b;
 }
+
+// Rows a float rotation of the ring's walk is advanced before its angles are evaluated afresh.
+// `each_row`: the rows whose other kernel, the generic one, evaluates every angle at its row.  Four
+// rows keep their dweight as near its 64-bit value (fp16 8192 x 2050, generic / 16 / 4 rows: off by
+// 2.0e-7 / 2.5e-7 / 1.8e-7 of it) at little cost (31.1 us both; 8192 x 4098, two chunks a thread, 53.2 /
+// 57.8).
+constexpr int rope_ring_anchor(bool each_row) { return each_row ? 4 : 16; }
 
 // Whether `slots` row slots walking `rows` rows (slot s: rows s, s + slots, ...) see positions
 // (row % seq) that only advance by `slots` or return to the walk's first one: slots is a

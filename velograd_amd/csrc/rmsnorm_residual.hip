@@ -271,6 +271,7 @@ struct BwdArgs {
   float rope_c_hi, rope_c_lo;  // kRopeG: log2(base) / half as an unevaluated float sum
   double rope_ratio;           // kRopeG: base^(-2/dim), one pair's frequency over the one before
   bool rope_back;              // the ring: a walk past a sequence's end returns to its first position
+  int32_t rope_anchor;         // the ring: rows between evaluations of a rotation afresh
 };
 
 // Output modes of the forward kernels.
@@ -2033,13 +2034,15 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_elem_kernel(cons
 // around a memory operation in the steady loop.  Each thread keeps the rotation (cos, sin) of
 // its pairs at the current row's position in float32 and advances it by S positions per row with
 // the rotation through S * freq_j (formed in double once per walk, rounded to float).  Where a
-// walk crosses the end of a sequence, S is a multiple or a divisor of rope_seq (rope_walk_ok: the
-// host plans this kernel only then, or when no walk reaches a sequence end), so the position
-// returns to the walk's first one and the rotation to its first value (kept in LDS with one
-// chunk per thread, evaluated afresh with two); a walk that goes kRopeAnchorRows rows without
-// such a return evaluates its angles afresh (double angle, exact reduction, float sincospi), so
-// no state is more than kRopeAnchorRows - 1 float steps from an exact value (about 3 * 2^-24 of
-// the pair per step).  The row group is a whole number of waves, so slots, rows and positions are
+// walk crosses the end of a sequence and S is a multiple or a divisor of rope_seq (rope_walk_ok,
+// a.rope_back), the position returns to the walk's first one and the rotation to its first value;
+// any other crossing evaluates the angles at the new position.  A walk that goes a.rope_anchor rows
+// without either evaluates its angles afresh (double angle, exact reduction, float cos and sin), so
+// no state is more than that less one float steps from an exact value (about 3 * 2^-24 of the pair
+// per step): 16 rows, or 4 where the general path forms every angle at its row (launch_plan.h:
+// rope_ring_anchor).  fp32 rows of ANY advance in double instead: their outputs hold what float
+// steps lose (dx 2.0e-7 off the 64-bit one against 0.7e-7, 4096 x 3002), and they are bound by HBM (40.7
+// / 40.6 us, 8192 x 2046).  The row group is a whole number of waves, so slots, rows and positions are
 // wave-uniform and the walk's bookkeeping is scalar.  The walk is bound by its vector
 // instructions as much as by HBM, so the row's decoded, rotated chunks stay in registers across
 // the reduction, the weight is decoded once, sums of products use fused multiply-adds, and for a
@@ -2054,19 +2057,23 @@ __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope
   constexpr int V = C::kVec;
   constexpr int P = V / 2;    // RoPE pairs per chunk
   constexpr int NP = NV * P;  // RoPE pairs per thread: pair e = k * P + q of chunk lt + k * tpr
-  // One chunk per thread keeps its pair frequencies and first rotations in LDS; with two, they
-  // would not fit 64 KiB beside the step rotations, so the frequencies are formed again where
-  // the angles are evaluated and the first rotation is evaluated afresh at a return.
-  constexpr bool kTablesInLds = NV == 1;
+  // The rotation state and step: float, or for fp32 rows of ANY double (see above).  One chunk per
+  // thread keeps its pair frequencies and first rotations in LDS; with two they would not fit 64 KiB
+  // beside the step rotations, so the first rotation is evaluated afresh at a return (also where the
+  // step is double), and the frequencies are formed again there, except for the 2-byte rows of ANY,
+  // which evaluate often.
+  constexpr bool kDoubleRot = ANY && DT == VELOGRAD_DTYPE_F32;
+  constexpr bool kFreqInLds = NV == 1 || (ANY && !kDoubleRot);
+  constexpr bool kFirstInLds = NV == 1 && !kDoubleRot;
+  using RotT = std::conditional_t<kDoubleRot, double, float>;
+  typedef RotT Rot2 __attribute__((ext_vector_type(2)));
   constexpr int PF = vg_plan::kRingPrefetch;
   constexpr int R = PF + 1;
-  constexpr int kRopeAnchorRows = 16;
   static_assert(NV == 1 || NV == 2, "the RoPE ring takes one or two chunks per thread");
   __shared__ float red[2][kMaxWavesPerRow];
-  // Dynamic LDS, pair-major so a wave reads consecutive 8-byte entries: with one chunk per thread
-  // each thread's pair frequencies (doubles), then step and first rotations (float pairs); with
-  // two, the step rotations only; then with several row groups dim floats for their combine
-  // (plan_bwd_rope_ring's lds_bytes).
+  // Dynamic LDS, pair-major so a wave reads consecutive entries: each thread's pair frequencies
+  // (doubles, kFreqInLds), its step rotations (Rot2), its first rotations (float pairs, kFirstInLds),
+  // then with several row groups dim floats for their combine (plan_bwd_rope_ring's lds_bytes).
   extern __shared__ __align__(16) float dyn_lds[];
 
   const int tpr = a.tpr;
@@ -2080,11 +2087,10 @@ __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope
   const int64_t pos0 = slot % seq;
   const int bd = blockDim.x;
   const int tid = threadIdx.x;
-  double* freq_lds = reinterpret_cast<double*>(dyn_lds);  // [P][bd], one chunk per thread
-  float2* step_lds = kTablesInLds ? reinterpret_cast<float2*>(freq_lds + P * bd)
-                                  : reinterpret_cast<float2*>(dyn_lds);  // [NP][bd]
-  float2* first_lds = step_lds + NP * bd;  // [P][bd], one chunk per thread
-  float* comb = reinterpret_cast<float*>(kTablesInLds ? first_lds + P * bd : first_lds);
+  double* freq_lds = reinterpret_cast<double*>(dyn_lds);  // [NP][bd], kFreqInLds
+  Rot2* step_lds = reinterpret_cast<Rot2*>(kFreqInLds ? freq_lds + NP * bd : freq_lds);  // [NP][bd]
+  float2* first_lds = reinterpret_cast<float2*>(step_lds + NP * bd);  // [P][bd], kFirstInLds
+  float* comb = reinterpret_cast<float*>(kFirstInLds ? first_lds + P * bd : first_lds);
   // 1 / dim is exact for a power of two, so s * (1 / dim) has the bits of s / dim
   const bool dim_pow2 = (a.dim & (a.dim - 1)) == 0;
   const float inv_dim = 1.0f / (float)a.dim;
@@ -2098,7 +2104,7 @@ __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope
   };
   // pair e's turns a position: base^(-2i/dim) / (2 pi), i its pair index in the row
   auto turns_of = [&](int e) {
-    if constexpr (kTablesInLds) return freq_lds[e * bd + tid];
+    if constexpr (kFreqInLds) return freq_lds[e * bd + tid];
     else
       return rope_freq(col_of(e / P) / 2 + e % P, a.rope_c_hi, a.rope_c_lo) * kInv2PiD;
   };
@@ -2126,25 +2132,28 @@ __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope
     const double rev = (double)S * g;
     double sv, cv;
     cos_sin_turn_d(rev - rint(rev), cv, sv);
-    step_lds[e * bd + tid] = float2{(float)cv, (float)sv};
-    if constexpr (kTablesInLds) {
-      freq_lds[e * bd + tid] = g;
+    step_lds[e * bd + tid] = Rot2{(RotT)cv, (RotT)sv};
+    if constexpr (kFreqInLds) freq_lds[e * bd + tid] = g;
+    if constexpr (kFirstInLds) {
       // the rotation at the walk's first position: double angle, reduced exactly, float cos and sin
       float s0, c0;
       cos_sin_turn(rope_frac((double)pos0 * g), c0, s0);
       first_lds[e * bd + tid] = float2{c0, s0};
     }
   }
-  float cr[NP], sr[NP];
+  RotT cr[NP], sr[NP];
   // the rotations at position p evaluated afresh: double angle, exact reduction, float cos and sin
   auto evaluate_at = [&](int64_t p) {
 #pragma unroll
     for (int e = 0; e < NP; ++e) {
-      cos_sin_turn(rope_frac((double)p * turns_of(e)), cr[e], sr[e]);
+      float c, sn;
+      cos_sin_turn(rope_frac((double)p * turns_of(e)), c, sn);
+      cr[e] = c;
+      sr[e] = sn;
     }
   };
   auto restore_first = [&]() {
-    if constexpr (kTablesInLds) {
+    if constexpr (kFirstInLds) {
 #pragma unroll
       for (int e = 0; e < NP; ++e) {
         const float2 f0 = first_lds[e * bd + tid];
@@ -2181,7 +2190,7 @@ __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope
       // inverse rotation of each pair (y0, y1) -> (y0 c + y1 s, y1 c - y0 s)
 #pragma unroll
       for (int q = 0; q < P; ++q) {
-        const float c = cr[k * P + q], sn = sr[k * P + q];
+        const float c = (float)cr[k * P + q], sn = (float)sr[k * P + q];
         const float g0 = gf[k][2 * q], g1 = gf[k][2 * q + 1];
         gf[k][2 * q] = __builtin_fmaf(g0, c, g1 * sn);
         gf[k][2 * q + 1] = __builtin_fmaf(g1, c, -(g0 * sn));
@@ -2214,28 +2223,28 @@ __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope
       }
     }
     // the next row's angles: the walk's first position again, evaluated afresh after
-    // kRopeAnchorRows - 1 steps, or one float step of S positions on (each thread reads only the
+    // a.rope_anchor rows, or one step of S positions on (each thread reads only the
     // LDS entries it wrote, in program order: no barrier)
     pos += S;
     ++since;
     if (pos >= seq) {
       since = 0;
       if (a.rope_back) {
+        if (!ANY || pos - S != pos0) restore_first();  // (a walk that has not left it keeps it)
         pos = pos0;
-        restore_first();
       } else {
         pos = (row + S) % seq;
         evaluate_at(pos);
       }
-    } else if (since == kRopeAnchorRows) {
+    } else if (since == a.rope_anchor) {
       since = 0;
       evaluate_at(pos);
     } else {
 #pragma unroll
       for (int e = 0; e < NP; ++e) {
-        const float2 st = step_lds[e * bd + tid];
-        const float cn = __builtin_fmaf(cr[e], st.x, -(sr[e] * st.y));
-        sr[e] = __builtin_fmaf(sr[e], st.x, cr[e] * st.y);
+        const Rot2 st = step_lds[e * bd + tid];
+        const RotT cn = __builtin_elementwise_fma(cr[e], st.x, -(sr[e] * st.y));
+        sr[e] = __builtin_elementwise_fma(sr[e], st.x, cr[e] * st.y);
         cr[e] = cn;
       }
     }
@@ -3344,6 +3353,7 @@ int32_t run_bwd(const void* grad_y, const void* saved, int32_t saved_is_h, const
   a.rope_c_lo = (float)(c - (double)a.rope_c_hi);
   a.rope_ratio = exp2(-c);
   a.rope_back = rope && vg_plan::rope_walk_ok(rows, slots, rope_seq);
+  a.rope_anchor = vg_plan::rope_ring_anchor(plan.any && !(aligned && dim % (16 / eb) == 0));
   VG_DISPATCH_TYPES(dtype, w_dtype, (launch_bwd<kD, kW>(a, saved_is_h != 0, rope, plan, st)));
   int32_t rc = check_launch(rope ? "velograd_rmsnorm_rope_bwd" : "velograd_rmsnorm_residual_bwd");
   if (rc != 0 || dweight == nullptr) return rc;
