@@ -484,6 +484,13 @@ int main() {
             plan_rope_tiles(16384, 4096, 4, 3, false).tile == 4,
         "whole tiles over short sequences");
   printf("rope tile plans checked: %ld\n", tiles);
+  // Ragged norm + RoPE backward rows: few short ones stay in the generic kernel.
+  CHECK(rope_bwd_generic_first(512, 74, 2, 256) && !rope_bwd_generic_first(1024, 510, 2, 256) &&
+            rope_bwd_generic_first(256, 514, 2, 256) && !rope_bwd_generic_first(257, 1002, 2, 256) &&
+            !rope_bwd_generic_first(1, 1026, 2, 256) && rope_bwd_generic_first(64, 130, 4, 256) &&
+            rope_bwd_generic_first(64, 258, 4, 256) && !rope_bwd_generic_first(65, 258, 4, 256) &&
+            !rope_bwd_generic_first(1, 514, 4, 256),
+        "generic-first norm + RoPE backward");
   // The allocation-free backward refuses fp32 2048 x 16384 (tests/test_zz_no_alloc.py): on 256
   // CUs with the default tuning, every plan the backward can pick for that shape (aligned or
   // not, with or without the ring) needs more partial rows than its 16 MiB scratch holds, while

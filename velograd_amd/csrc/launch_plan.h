@@ -586,6 +586,17 @@ inline BwdPlan plan_bwd_rope_ring_any(int64_t rows, int64_t dim, int elem_bytes,
 // 57.8).
 constexpr int rope_ring_anchor(bool each_row) { return each_row ? 4 : 16; }
 
+// Whether such rows of a short tensor stay in the generic kernel: the ring's set-up of each pair's
+// rotation and its combine of many row groups outlast a few short rows.  Measured (generic / ring, us):
+// bf16 74 at 16 rows 5.6 / 9.2, 512 7.8 / 9.8, 1024 10.1 / 10.0; 510 at 512 9.5 / 10.6, 1024 13.0 / 10.9;
+// 514 at 64 rows 7.8 / 8.9, 256 8.0 / 9.2, 512 10.4 / 9.6; 2050 at 1 row 9.6 / 8.2; fp32 130 at 64 rows
+// 6.5 / 7.2, 512 8.4 / 7.6; 258 at 16 rows 5.9 / 6.9, 128 8.1 / 7.1; 514 at 16 rows 6.7 / 6.6.
+inline bool rope_bwd_generic_first(int64_t rows, int64_t dim, int elem_bytes, int cus) {
+  const int64_t V = 16 / elem_bytes, waves = ((dim + V - 1) / V + kWave - 1) / kWave;
+  if (waves == 1) return elem_bytes == 2 ? rows < 4 * (int64_t)cus : rows <= cus;
+  return waves == 2 && rows <= (elem_bytes == 2 ? cus : cus / 4);
+}
+
 // Whether `slots` row slots walking `rows` rows (slot s: rows s, s + slots, ...) see positions
 // (row % seq) that only advance by `slots` or return to the walk's first one: slots is a
 // multiple or a divisor of seq, or no walk reaches the end of a sequence.

@@ -2684,7 +2684,10 @@ BwdPlan plan_bwd(int64_t rows, int64_t dim, int elem_bytes, bool aligned, bool a
     const BwdPlan r = vg_plan::plan_bwd_rope_ring(rows, dim, elem_bytes, aligned, cus);
     if (r.ring) return r;
     const BwdPlan ra = vg_plan::plan_bwd_rope_ring_any(rows, dim, elem_bytes, cus);
-    if (ra.ring && aligned_elem) return ra;
+    const bool whole = aligned && dim % (16 / elem_bytes) == 0;  // (bwd_vec_kernel's otherwise)
+    if (ra.ring && aligned_elem &&
+        (whole || !vg_plan::rope_bwd_generic_first(rows, dim, elem_bytes, cus)))
+      return ra;
   }
   if (rope)
     return vg_plan::plan_bwd_rope(rows, dim, elem_bytes, aligned, cus, t.bwd_nv, t.bwd_block,
