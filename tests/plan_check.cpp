@@ -5,6 +5,7 @@
 //     wave64s per row, and its workgroup fits the kernel's launch bound for that NV;
 //   * the backward's workgroups, LDS and partial rows fit the workspace the size query reports.
 #include <algorithm>
+#include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
 
@@ -491,6 +492,23 @@ int main() {
             rope_bwd_generic_first(64, 258, 4, 256) && !rope_bwd_generic_first(65, 258, 4, 256) &&
             !rope_bwd_generic_first(1, 514, 4, 256),
         "generic-first norm + RoPE backward");
+  // A RoPE pair's turns a position have the same bits in both chunks that hold it: the row's last
+  // chunk begins at dim - V, mostly inside the one before it.
+  for (int eb = 2; eb <= 4; eb += 2) {
+    const int V = 16 / eb, P = V / 2;
+    for (int dim = V + 2; dim < 4200; dim += dim < 64 ? 2 : 38) {
+      const double c = log2(1e4) / (dim / 2), ratio = exp2(-c);
+      auto first = [&](int i) { return exp2(-i * c) * 0.15915494309189535; };
+      auto turns = [&](int col, int i) {  // pair i's in the lane whose chunk begins at col
+        double g = rope_first_turns(col / 2, P, ratio, first);
+        for (int q = col / 2; q < i; ++q) g *= ratio;
+        return g;
+      };
+      const int last = (dim - 1) / V;  // chunk
+      for (int i = (dim - V) / 2; i < last * P; ++i)
+        CHECK(turns((last - 1) * V, i) == turns(dim - V, i), "pair %d of %d", i, dim);
+    }
+  }
   // The allocation-free backward refuses fp32 2048 x 16384 (tests/test_zz_no_alloc.py): on 256
   // CUs with the default tuning, every plan the backward can pick for that shape (aligned or
   // not, with or without the ring) needs more partial rows than its 16 MiB scratch holds, while

@@ -579,6 +579,17 @@ inline BwdPlan plan_bwd_rope_ring_any(int64_t rows, int64_t dim, int elem_bytes,
   return b;
 }
 
+// The turns a position of RoPE pair i, the first of a lane's chunk: `first` at the pair that begins the
+// row's aligned chunk of `pairs` around it, then the double ratio from pair to pair (as the lane goes on
+// to its next ones).  So the pairs that the row's last chunk shares with the one before it, where it
+// begins inside that, have the same bits in both lanes, and so have the columns that both store.
+template <typename First>
+VG_HOST_DEVICE inline double rope_first_turns(int i, int pairs, double ratio, First first) {
+  double g = first(i - i % pairs);
+  for (int t = i % pairs; t > 0; --t) g *= ratio;
+  return g;
+}
+
 // Rows a float rotation of the ring's walk is advanced before its angles are evaluated afresh.
 // `each_row`: the rows whose other kernel, the generic one, evaluates every angle at its row.  Four
 // rows keep their dweight as near its 64-bit value (fp16 8192 x 2050, generic / 16 / 4 rows: off by

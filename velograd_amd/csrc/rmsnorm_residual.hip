@@ -2127,8 +2127,12 @@ __global__ __launch_bounds__(vg_plan::kRingBlock, NV == 1 ? 4 : 2) void bwd_rope
   double g = 0.0;
 #pragma unroll 1
   for (int e = 0; e < NP; ++e) {
-    g = e % P == 0 ? rope_freq(col_of(e / P) / 2, a.rope_c_hi, a.rope_c_lo) * kInv2PiD
-                   : g * a.rope_ratio;
+    if (e % P == 0)
+      g = vg_plan::rope_first_turns(
+          col_of(e / P) / 2, ANY ? P : 1, a.rope_ratio,
+          [&](int i) { return rope_freq(i, a.rope_c_hi, a.rope_c_lo) * kInv2PiD; });
+    else
+      g = g * a.rope_ratio;
     const double rev = (double)S * g;
     double sv, cv;
     cos_sin_turn_d(rev - rint(rev), cv, sv);
