@@ -289,21 +289,27 @@ Tensors norm_rope_backward(const at::Tensor& g, const at::Tensor& h, const OptTe
 
 PYBIND11_MODULE(_fastpath, m) {
   m.doc() = "C++ fast path of the kernels' common calls, for launch-bound sizes";
-  m.def("forward", &forward, "forward(x, residual, weight, eps, min_mean_sq) -> [y, h, inv_rms]",
-        pybind11::arg("x"), pybind11::arg("residual"), pybind11::arg("weight"),
-        pybind11::arg("eps"), pybind11::arg("min_mean_sq"));
-  m.def("forward_quantised", &forward_quantised, pybind11::arg("x"), pybind11::arg("residual"),
-        pybind11::arg("weight"), pybind11::arg("eps"), pybind11::arg("mx_format"));
-  m.def("backward", &backward, pybind11::arg("grad_out"), pybind11::arg("saved"),
+  // Allocation and launch run without the interpreter lock, as torch's own calls do: either may
+  // wait (for memory, for room in the queue), and other Python threads go on meanwhile.
+  using NoGil = pybind11::call_guard<pybind11::gil_scoped_release>;
+  m.def("forward", &forward, NoGil(),
+        "forward(x, residual, weight, eps, min_mean_sq) -> [y, h, inv_rms]", pybind11::arg("x"),
+        pybind11::arg("residual"), pybind11::arg("weight"), pybind11::arg("eps"),
+        pybind11::arg("min_mean_sq"));
+  m.def("forward_quantised", &forward_quantised, NoGil(), pybind11::arg("x"),
+        pybind11::arg("residual"), pybind11::arg("weight"), pybind11::arg("eps"),
+        pybind11::arg("mx_format"));
+  m.def("backward", &backward, NoGil(), pybind11::arg("grad_out"), pybind11::arg("saved"),
         pybind11::arg("weight"), pybind11::arg("inv_rms"), pybind11::arg("saved_is_h"),
         pybind11::arg("dresidual_out"), pybind11::arg("grad_h"));
-  m.def("rope", &rope, pybind11::arg("q"), pybind11::arg("k"), pybind11::arg("head_dim"),
-        pybind11::arg("theta"), pybind11::arg("inverse"));
-  m.def("rope_interleaved", &rope_interleaved, pybind11::arg("x"), pybind11::arg("base"),
-        pybind11::arg("inverse"));
-  m.def("norm_rope", &norm_rope, pybind11::arg("x"), pybind11::arg("residual"),
+  m.def("rope", &rope, NoGil(), pybind11::arg("q"), pybind11::arg("k"),
+        pybind11::arg("head_dim"), pybind11::arg("theta"), pybind11::arg("inverse"));
+  m.def("rope_interleaved", &rope_interleaved, NoGil(), pybind11::arg("x"),
+        pybind11::arg("base"), pybind11::arg("inverse"));
+  m.def("norm_rope", &norm_rope, NoGil(), pybind11::arg("x"), pybind11::arg("residual"),
         pybind11::arg("weight"), pybind11::arg("eps"), pybind11::arg("base"),
         pybind11::arg("min_mean_sq"));
-  m.def("norm_rope_backward", &norm_rope_backward, pybind11::arg("grad_y"), pybind11::arg("h"),
-        pybind11::arg("weight"), pybind11::arg("inv_rms"), pybind11::arg("base"));
+  m.def("norm_rope_backward", &norm_rope_backward, NoGil(), pybind11::arg("grad_y"),
+        pybind11::arg("h"), pybind11::arg("weight"), pybind11::arg("inv_rms"),
+        pybind11::arg("base"));
 }
