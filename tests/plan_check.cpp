@@ -385,15 +385,6 @@ int main() {
     CHECK(fwd_late_h(p) == (dim <= 4096), "fwd_late_h dim=%lld tpr=%d", (long long)dim, p.tpr);
   }
   CHECK(!fwd_late_h(plan_rows(4096, 2, false, 0, kFwdOrder)), "fwd_late_h on the generic plan");
-  // the norm + RoPE forward's walk length: 32 rows for row groups of more than 256 threads over
-  // at least 16384 rows, else 16; the walk's inv_rms stores need a thread per row of the walk
-  for (int tpr = 64; tpr <= 1024; tpr += 64) {
-    for (int64_t rows : {1, 15, 16, 4096, 16383, 16384, 16385, 262147}) {
-      const int w = fwd_rope_walk_rows(rows, tpr);
-      CHECK(w == ((tpr > 256 && rows >= 16384) ? 32 : 16) && w <= tpr,
-            "fwd_rope_walk_rows rows=%lld tpr=%d -> %d", (long long)rows, tpr, w);
-    }
-  }
   // Wide norm + RoPE rows (tests/test_gpu_rmsnorm_rope.py): the backward's walk takes three
   // chunks per thread up to 1536 chunks; past that the plain plan with each pair's rotation
   // evaluated directly, two chunks per thread in 832-thread rows at 1540 chunks and four in
@@ -509,6 +500,63 @@ int main() {
         CHECK(turns((last - 1) * V, i) == turns(dim - V, i), "pair %d of %d", i, dim);
     }
   }
+  // Rows of any length: every column in the row group's lanes (the forward's at most 2 V - 2 stray
+  // elements, one to a lane), workgroups, LDS and partial rows within their bounds, the norm + RoPE
+  // ring's LDS as its kernel lays it out, and never more partial rows than the generic kernel's,
+  // whose no-alloc limit wide rows keep.
+  long any = 0;
+  for (int64_t dim = 1; dim <= 16500; dim += dim < 80 ? 1 : dim < 2100 ? 13 : 211) {
+    for (int eb = 2; eb <= 4; eb += 2) {
+      const int V = 16 / eb, P = V / 2;
+      for (int form = 0; form < 4; ++form) {
+        const RowPlan p = plan_any_rows(dim, eb, form & 1, form & 2);
+        const bool wide_one_stream = form == 0 && dim / V > kAnyOneStreamChunks;
+        CHECK(p.vec == (dim >= V && dim / V <= 2048 && !wide_one_stream), "any rows at %lld x %d",
+              (long long)dim, eb);
+        if (!p.vec) continue;
+        ++any;
+        CHECK(row_plan_valid(p, dim / V * V, eb) && p.block <= max_block_for_nv(p.nv) &&
+                  (int64_t)p.nv * p.tpr >= dim / V && p.tpr >= 2 * V - 2,
+              "any-row forward at %lld x %d", (long long)dim, eb);
+      }
+      for (int64_t rows : {1, 7, 300, 16384}) {
+        for (int cus : {1, 64, 256}) {
+          const size_t ws = bwd_workspace_bytes(rows, dim, cus, 0, 1024, 16);
+          const BwdPlan b = plan_bwd_ring_any(rows, dim, eb, cus);
+          const int64_t chunks = (dim + V - 1) / V;
+          CHECK(b.ring == (dim >= V && chunks <= 2 * kRingBlock), "ring over %lld x %d",
+                (long long)dim, eb);
+          if (b.ring) {
+            CHECK(b.any && (int64_t)b.rp.nv * b.rp.tpr >= chunks && b.rp.tpr % kWave == 0 &&
+                      b.rp.nv >= 1 && b.rp.nv <= kRingMaxNV &&
+                      b.rp.block == b.rp.tpr * b.rp.groups && b.rp.block <= kRingBlock &&
+                      b.wgs >= 1 && b.wgs <= cus && (b.wgs - 1) * b.rp.groups < rows &&
+                      b.lds_bytes == (b.rp.groups > 1 ? (size_t)dim * sizeof(float) : 0) &&
+                      (size_t)b.wgs * dim * sizeof(float) <= ws,
+                  "any-row ring %lld x %lld x %d", (long long)rows, (long long)dim, eb);
+            for (int waves : {1, 16, 64})
+              CHECK(plan_bwd(rows, dim, eb, false, cus, 0, 1024, waves).wgs >= b.wgs,
+                    "fewer generic partial rows at %lld", (long long)dim);
+          }
+          const BwdPlan r = plan_bwd_rope_ring_any(rows, dim, eb, cus);
+          CHECK(r.ring == (dim >= V && dim % 2 == 0 && chunks <= 2 * kRingBlock),
+                "norm + RoPE ring over %lld x %d", (long long)dim, eb);
+          if (r.ring) {
+            const size_t pairs = (size_t)r.rp.block * r.rp.nv * P;
+            const size_t tables = r.rp.nv == 1 ? 24 * pairs : 16 * pairs;
+            CHECK(r.any && (int64_t)r.rp.nv * r.rp.tpr >= chunks && r.rp.tpr % kWave == 0 &&
+                      r.rp.block == r.rp.tpr * r.rp.groups && r.rp.block <= kRingBlock &&
+                      r.wgs >= 1 && r.wgs <= cus * kRopeRingMaxWgsPerCu &&
+                      r.lds_bytes == tables + (r.rp.groups > 1 ? (size_t)dim * 4 : 0) &&
+                      r.lds_bytes <= 64 * 1024 && (size_t)r.wgs * dim * sizeof(float) <= ws,
+                  "any-row norm + RoPE ring %lld x %lld x %d: lds %zu", (long long)rows,
+                  (long long)dim, eb, r.lds_bytes);
+          }
+        }
+      }
+    }
+  }
+  printf("any-row plans checked: %ld\n", any);
   // The allocation-free backward refuses fp32 2048 x 16384 (tests/test_zz_no_alloc.py): on 256
   // CUs with the default tuning, every plan the backward can pick for that shape (aligned or
   // not, with or without the ring) needs more partial rows than its 16 MiB scratch holds, while

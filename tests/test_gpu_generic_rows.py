@@ -1,9 +1,10 @@
-"""Rows that are not 16-byte multiples (hidden sizes such as 4100 bf16).  Rows of 8n + 4
-two-byte elements whose streams start on 8-byte boundaries take the register-resident kernels
-(whole chunks in 8-byte halves, the last 4 elements a half chunk); the others take the generic
-kernels: each row's 16-byte-aligned middle moves in 16-byte accesses and its head and tail
-element by element, and the backward sums its dweight columns in LDS, where a column moves
-between threads from row to row.  Checked against the oracle with tests/_parity.py's tolerances: contiguous
+"""Rows that are not 16-byte multiples (hidden sizes such as 4100 bf16), in the kernels that the
+planner gives them: the forward in chunks from any element; the backward of 8n + 4 two-byte elements
+on 8-byte boundaries in whole chunks of 8-byte halves with a half chunk at the end, of other rows in
+chunks from any element or element by element; and, past the registers, the generic kernels, which
+move each row's 16-byte-aligned middle in 16-byte accesses and its head and tail element by element,
+the backward summing its dweight columns in LDS, where a column moves between threads from row to
+row.  Checked against the oracle with tests/_parity.py's tolerances: contiguous
 tensors (every row through the aligned middle), tensors of different row strides (rows whose
 streams disagree inside a 16-byte line take the element-wise path, so one workgroup mixes both),
 rows at the LDS limit and past it, and bitwise repeatability of dx and dweight."""
@@ -29,8 +30,8 @@ CASES = [
     (777, 16000, BF16, "same", False),   # LDS sums at their limit (kGenericLdsCols)
     (300, 16008, BF16, "same", True),    # past it: element-wise rows, sums in the partial row
     (64, 20002, F32, "same", False),
-    # rows of 8n + 4 two-byte elements on 8-byte boundaries: the register-resident kernels over
-    # the whole chunks in 8-byte halves plus a half chunk (fwd_vec_kernel X8, bwd_ring_kernel
+    # rows of 8n + 4 two-byte elements on 8-byte boundaries: the forward in chunks from any element,
+    # the backward in whole chunks of 8-byte halves plus a half chunk (bwd_ring_kernel
     # kRing8), down to one whole chunk (dim 12)
     (999, 2052, F16, "f32", False),
     (4097, 1028, BF16, None, True),

@@ -5,7 +5,9 @@
 // register-resident kernels give each row `tpr` threads (whole wave64s) and each thread NV
 // chunks, c = lane + k * tpr for k < NV, so that consecutive lanes touch consecutive 16-byte
 // chunks (coalesced 1 KiB per wave instruction).  Rows whose length is not a multiple of the
-// chunk, misaligned rows, and rows too long for registers use the generic looping kernels.
+// chunk and misaligned rows go in chunks from any element (plan_any_rows, plan_bwd_ring_any,
+// plan_bwd_rope_ring_any, plan_rope_tiles) or, short ones, element by element; rows too long for
+// registers, and the few that these rules leave, use the generic looping kernels.
 #ifndef VELOGRAD_LAUNCH_PLAN_H
 #define VELOGRAD_LAUNCH_PLAN_H
 
@@ -453,7 +455,7 @@ inline BwdPlan plan_bwd_ring_any(int64_t rows, int64_t dim, int elem_bytes, int 
 // 31.8, and 3001 and 4095 alike.
 constexpr int kRingElemMaxM = 8;
 
-inline int elem_per_lane(int64_t dim) {
+constexpr int elem_per_lane(int64_t dim) {
   if (dim <= 0 || dim > (int64_t)kRingElemMaxM * kRingBlock) return 0;
   return dim > 512 ? 8 : 4;
 }
@@ -505,8 +507,9 @@ inline BwdPlan plan_bwd_ring_elem(int64_t rows, int64_t dim, int elem_bytes, int
 // of one 16-byte chunk per thread where a row has at most kRingBlock chunks (its rotation state
 // and tables keep it at 128 VGPRs), else of two (rows of up to 2 * kRingBlock chunks; 256
 // VGPRs), row groups packed into workgroups of up to kRingBlock threads, rope_ring_wgs_per_cu of
-// them per CU.  `ring` is false when the row layout does not suit it.  The kernel also needs every
-// slot's walk to advance by the slot count or return to its first position (rope_walk_ok).
+// them per CU.  `ring` is false when the row layout does not suit it.  Where a slot's walk does not just
+// advance by the slot count or return to its first position (rope_walk_ok), the kernel evaluates its
+// angles afresh at each sequence it enters.
 constexpr int kRopeRingMaxWgsPerCu = 2;
 
 // One chunk per thread: one workgroup per CU when it fills kRingBlock threads (eight waves),
@@ -737,15 +740,6 @@ VG_HOST_DEVICE inline RopeTile rope_tile(uint32_t i, uint32_t rows, uint32_t seq
   t.step = across ? seq : 1;
   t.n = (int)(cut - at < (uint32_t)r ? cut - at : (uint32_t)r);
   return t;
-}
-
-// Rows a workgroup walked in the strided norm + RoPE forward that fwd_rope_tile_kernel replaced
-// (no kernel takes it any more; the planner's test still states it).
-constexpr int kNormRopeRows = 16;
-constexpr int kNormRopeLongRows = 32;
-constexpr int64_t kNormRopeLongMinRows = 16384;
-inline int fwd_rope_walk_rows(int64_t rows, int tpr) {
-  return tpr > 256 && rows >= kNormRopeLongMinRows ? kNormRopeLongRows : kNormRopeRows;
 }
 
 // Workspace of the backward's dweight partial rows.  The plan depends on the element size, on

@@ -297,7 +297,7 @@ __device__ __forceinline__ double rope_freq(int i, float c_hi, float c_lo) {
 
 // A double angle in revolutions reduced exactly to [-1/2, 1/2], and the cos and sin of such an
 // angle: the quarter turn nearest to it, then the Taylor series of sin and cos over the +-1/8
-// turn that is left (0.72 and 0.98 ulp at most against 64 bits over 4 million angles; the leading
+// turn that is left (1.02 ulp at most against 64 bits over 20 million angles; the leading
 // pi/2 in two floats).
 __device__ __forceinline__ float rope_frac(double rev) { return (float)(rev - rint(rev)); }
 __device__ __forceinline__ void cos_sin_turn(float rev, float& c, float& s) {
@@ -949,6 +949,7 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_rope_tile_kernel(con
 // output) only; longer rows move in chunks (fwd_vec_kernel's ANY).
 // ------------------------------------------------------------------------------------------
 constexpr int64_t kFwdElemMaxDim = 64;  // the host plans it for rows of at most this length
+constexpr int kFwdElemPerLane = vg_plan::elem_per_lane(kFwdElemMaxDim);
 
 template <int DT, int WDT, int M>
 __global__ __launch_bounds__(vg_plan::kRingBlock) void fwd_elem_kernel(const FwdArgs a) {
@@ -1025,10 +1026,10 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void fwd_elem_kernel(const Fwd
 }
 
 // ------------------------------------------------------------------------------------------
-// Forward, the rows that the kernels above do not take (longer than their registers hold, wide any
-// rows without a residual (plan_any_rows), rows shorter than a chunk with a quantised or RoPE
-// output, streams off their element's alignment): one row per workgroup, two passes over the row (the second
-// re-reads x and residual, normally from L2, and recomputes the identical fp32 h).
+// Forward, the rows that the kernels above do not take (longer than their registers hold, wide
+// ragged ones without a residual (plan_any_rows), rows shorter than a chunk with a quantised or RoPE
+// output, streams off their element's alignment): one row per workgroup, two passes over the row
+// (the second re-reads x and residual, normally from L2, and recomputes the identical fp32 h).
 // ------------------------------------------------------------------------------------------
 template <int DT, int WDT, int OUT>
 __global__ __launch_bounds__(kGenericBlock) void fwd_generic_kernel(const FwdArgs a) {
@@ -2027,10 +2028,11 @@ __global__ __launch_bounds__(vg_plan::kRingBlock) void bwd_ring_elem_kernel(cons
 }
 
 // ------------------------------------------------------------------------------------------
-// Backward with the fused RoPE gradient, ring-pipelined (launch_plan.h: plan_bwd_rope_ring):
-// whole rows of NV (1 or 2) 16-byte chunks per thread, the saved tensor h, no grad_h or dres (the
-// module's backward).  The walk, ring and steady loop are bwd_ring_kernel's: slot s walks rows
-// s, s + S, ... (S slots), three row buffers, rows past the end read the last row, no branch
+// Backward with the fused RoPE gradient, ring-pipelined (launch_plan.h: plan_bwd_rope_ring, and with
+// ANY plan_bwd_rope_ring_any: even rows of any length, streams at any element, the row's last chunk
+// overlapping the one before it): NV (1 or 2) 16-byte chunks per thread, the saved tensor h, no
+// grad_h or dres (the module's backward).  The walk, ring and steady loop are bwd_ring_kernel's: slot
+// s walks rows s, s + S, ... (S slots), three row buffers, rows past the end read the last row, no branch
 // around a memory operation in the steady loop.  Each thread keeps the rotation (cos, sin) of
 // its pairs at the current row's position in float32 and advances it by S positions per row with
 // the rotation through S * freq_j (formed in double once per walk, rounded to float).  Where a
@@ -2670,10 +2672,8 @@ RowPlan plan_fwd(int64_t dim, int elem_bytes, bool aligned, bool one_stream, boo
 // `aligned8`: every stream starts on an 8-byte boundary (the weight on a 16-byte one), the
 // condition of the ring's kRing8 rows; `aligned_elem`: on their own elements' (kRingAny).
 BwdPlan plan_bwd(int64_t rows, int64_t dim, int elem_bytes, bool aligned, bool aligned8,
-                 bool aligned_elem, bool has_gh, bool dx_is_gh, int cus, bool rope,
-                 int64_t rope_seq) {
+                 bool aligned_elem, bool has_gh, bool dx_is_gh, int cus, bool rope) {
   const Tuning& t = tuning();
-  (void)rope_seq;
   if (!rope && t.bwd_ring) {
     const BwdPlan r = vg_plan::plan_bwd_ring(rows, dim, elem_bytes, aligned, cus, t.bwd_nv,
                                              t.ring_block, t.ring_wgs_per_cu);
@@ -2820,14 +2820,11 @@ void launch_rope_tiles(const FwdArgs& a, const vg_plan::RopeTilePlan& p, bool an
   }
 }
 
-// Rows of element-strided lanes (fwd_elem_kernel): `p` from plan_elem_rows, m elements a lane.
+// Rows of element-strided lanes (fwd_elem_kernel): `p` from plan_elem_rows.
 template <int DT, int WDT>
-void launch_fwd_elem(const FwdArgs& a, const RowPlan& p, int m, hipStream_t st) {
+void launch_fwd_elem(const FwdArgs& a, const RowPlan& p, hipStream_t st) {
   const dim3 grid((uint32_t)((a.rows + p.groups - 1) / p.groups)), block(p.block);
-  if (m == 4)
-    hipLaunchKernelGGL((fwd_elem_kernel<DT, WDT, 4>), grid, block, 0, st, a);
-  else
-    hipLaunchKernelGGL((fwd_elem_kernel<DT, WDT, 8>), grid, block, 0, st, a);
+  hipLaunchKernelGGL((fwd_elem_kernel<DT, WDT, kFwdElemPerLane>), grid, block, 0, st, a);
 }
 
 template <int DT, int WDT, int F>
@@ -3195,7 +3192,7 @@ int32_t run_fwd(const char* what, int out, const void* x, const void* residual,
       if (any)
         VG_DISPATCH_TYPES(dtype, w_dtype, (launch_fwd_any<kD, kW, kOutDtype>(a, p, st)));
       else if (elem_m > 0)
-        VG_DISPATCH_TYPES(dtype, w_dtype, (launch_fwd_elem<kD, kW>(a, p, elem_m, st)));
+        VG_DISPATCH_TYPES(dtype, w_dtype, (launch_fwd_elem<kD, kW>(a, p, st)));
       else
         VG_DISPATCH_TYPES(dtype, w_dtype, (launch_fwd<kD, kW, kOutDtype>(a, p, st)));
       break;
@@ -3273,7 +3270,7 @@ int32_t run_bwd(const void* grad_y, const void* saved, int32_t saved_is_h, const
                             elem_ok_ptr(dx, eb) && elem_ok_ptr(dres, eb) &&
                             elem_ok_ptr(grad_h, eb) && elem_ok_ptr(weight, elem_bytes_of(w_dtype));
   BwdPlan plan = plan_bwd(rows, dim, eb, aligned, aligned8, aligned_elem, grad_h != nullptr,
-                          dx == grad_h, cus, rope, rope_seq);
+                          dx == grad_h, cus, rope);
   // the columns the row plan lays out
   const int64_t plan_dim = plan.x8    ? dim - 4
                            : plan.any ? (dim + 16 / eb - 1) / (16 / eb) * (16 / eb)
@@ -3308,7 +3305,8 @@ int32_t run_bwd(const void* grad_y, const void* saved, int32_t saved_is_h, const
     size_t need = (size_t)plan.wgs * (size_t)dim * sizeof(float);
     if (static_scratch) {
       // velograd_rmsnorm_residual_bwd_noalloc: the partial rows go to the library's own array.
-      // Wide rows that the chunked kernels cannot take are held to the generic kernel's need.
+      // Wide rows that the chunked kernels cannot take are held to the generic kernel's need, which
+      // is never less than the plan's (it has at least one workgroup a CU or a row).
       if (plan.any && dim > vg_plan::kRingElemMaxM * vg_plan::kRingBlock)
         need = (size_t)vg_plan::plan_bwd(rows, dim, eb, false, cus, tuning().bwd_nv,
                                          tuning().bwd_block, tuning().bwd_waves_per_cu).wgs *
