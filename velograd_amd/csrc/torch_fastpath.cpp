@@ -285,13 +285,23 @@ Tensors norm_rope_backward(const at::Tensor& g, const at::Tensor& h, const OptTe
   return {b.dx, b.dweight};
 }
 
+// The interpreter lock given up for a scope (pybind11's own guard looks its internals up as well, a
+// tenth of a microsecond a call).
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  Unlocked() = default;
+  Unlocked(const Unlocked&) = delete;
+  Unlocked& operator=(const Unlocked&) = delete;
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
 }  // namespace
 
 PYBIND11_MODULE(_fastpath, m) {
   m.doc() = "C++ fast path of the kernels' common calls, for launch-bound sizes";
   // Allocation and launch run without the interpreter lock, as torch's own calls do: either may
   // wait (for memory, for room in the queue), and other Python threads go on meanwhile.
-  using NoGil = pybind11::call_guard<pybind11::gil_scoped_release>;
+  using NoGil = pybind11::call_guard<Unlocked>;
   m.def("forward", &forward, NoGil(),
         "forward(x, residual, weight, eps, min_mean_sq) -> [y, h, inv_rms]", pybind11::arg("x"),
         pybind11::arg("residual"), pybind11::arg("weight"), pybind11::arg("eps"),
