@@ -1,6 +1,7 @@
 """The register-resident forward issues all of a row's loads before it waits for any of them: its
 gfx950 assembly (hipcc, no GPU needed) holds no wait on vector memory between the first load and
-the last one of a row.  A wait there costs 2-10% of the pass and shows in no result."""
+the last one of a row.  A wait there costs 2-10% of the pass and shows in no result.  (An fp32 weight
+beside 2-byte activations, with two or more chunks a thread, is loaded after the wait on purpose.)"""
 
 import os
 import re
@@ -20,12 +21,14 @@ CHUNKS, ANY_NO_RES = 0, 2
 # dtype, weight dtype, chunks a thread, output, rows
 KERNELS = [(BF16, BF16, nv, out, CHUNKS) for nv in (1, 2, 3, 4)
            for out in (DTYPE, DTYPE_LATE_H, FP8, MXFP8, MXFP4)]
-KERNELS += [(F16, F32, 2, FP8, CHUNKS), (F32, F32, 2, DTYPE, CHUNKS)]
+KERNELS += [(F16, F32, 2, FP8, CHUNKS), (BF16, F32, 2, DTYPE, CHUNKS), (BF16, F32, 1, DTYPE, CHUNKS),
+            (F32, F32, 2, DTYPE, CHUNKS)]
 KERNELS += [(BF16, BF16, 1, out, ANY_NO_RES) for out in (FP8, MXFP8, MXFP4)]
 
 
-def _early_waits(body):
-    """The waits between the first and the last of the loads before the first store or barrier."""
+def _early_waits(body, weight_late):
+    """The waits between the first and the last of the loads before the first store or barrier;
+    `weight_late`: of the activations' (non-temporal) alone."""
     seq = []
     for line in body:
         line = line.strip()
@@ -33,7 +36,8 @@ def _early_waits(body):
             break
         if line.startswith("global_load") or (line.startswith("s_waitcnt") and "vmcnt" in line):
             seq.append(line)
-    loads = [i for i, line in enumerate(seq) if line.startswith("global_load")]
+    loads = [i for i, line in enumerate(seq)
+             if line.startswith("global_load") and (not weight_late or line.split()[-1] == "nt")]
     assert len(loads) >= 2, seq
     return [line for line in seq[:loads[-1]] if line.startswith("s_waitcnt")]
 
@@ -62,5 +66,5 @@ def test_no_wait_between_a_rows_loads(tmp_path):
         elif name is not None:
             bodies[name].append(line)
     assert set(KERNELS) <= set(bodies)
-    early = {k: _early_waits(bodies[k]) for k in KERNELS}
+    early = {k: _early_waits(bodies[k], k[0] != F32 and k[1] == F32 and k[2] > 1) for k in KERNELS}
     assert not any(early.values()), {k: w for k, w in early.items() if w}

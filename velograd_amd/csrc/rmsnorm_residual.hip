@@ -517,10 +517,17 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
       xv[k] = load_chunk(a.x, rw * a.ld_x + col[k]);
       if (has_res) rv[k] = load_chunk(a.res, rw * a.ld_res + col[k]);
     }
-    if (has_w) {
+    auto load_w = [&]() {
+      if (!has_w) return;
 #pragma unroll
       for (int k = 0; k < NV; ++k) wc[k].load(a.w, col[k]);
-    }
+    };
+    // An fp32 weight beside 2-byte activations is twice their bytes, all from L2: with two or more
+    // chunks a thread it goes out after the wait, while the row is summed (fp32 weight, with the
+    // others / after, us: without a residual 8192 x 12288 82.5 / 71.9, 16384 x 4096 49.6 / 47.8, to fp8
+    // 8192 x 16384 208.8 / 195.5, 16384 x 5120 101.2 / 97.3; 32768 x 1024 39.4 / 39.9).
+    constexpr bool kLateW = WeightChunk<DT, WDT>::kParts > 1 && NV > 1;
+    if constexpr (!kLateW) load_w();
     // one wait for all of them, before the first store of h: a wait after that, at the next
     // chunk's first use, would be for the store as well
 #pragma unroll
@@ -528,6 +535,7 @@ __global__ __launch_bounds__(max_block_for_nv(NV)) void fwd_vec_kernel(const Fwd
       forget(xv[k]);
       forget(rv[k]);
     }
+    if constexpr (kLateW) load_w();
   }
 
   auto make_h = [&](int k, float* hf) {
