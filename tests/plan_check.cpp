@@ -410,14 +410,17 @@ int main() {
   }
   // Forward rows of any length with a residual: two chunks a thread in up to two waves, else one.
   for (int64_t dim : {1001, 2047, 2055, 2056, 2201, 3002, 3076, 4095}) {
-    const RowPlan p = plan_any_rows(dim, 2, true, false);
+    const RowPlan p = plan_any_rows(16384, dim, 2, true, false);
     CHECK(p.vec && p.nv == (dim < 2056 ? 2 : 1), "any-row forward at %lld: nv %d", (long long)dim,
           p.nv);
   }
-  // Without one, plain rows of more than 896 chunks keep the generic kernel.
-  CHECK(plan_any_rows(7175, 2, false, false).vec && !plan_any_rows(7176, 2, false, false).vec &&
-            !plan_any_rows(4095, 4, false, false).vec && !plan_any_rows(14001, 2, false, false).vec &&
-            plan_any_rows(14001, 2, true, false).vec && plan_any_rows(14001, 2, false, true).vec,
+  // Without one, plain rows of more than 896 chunks keep the generic kernel past 512 of them.
+  CHECK(plan_any_rows(16384, 7175, 2, false, false).vec &&
+            !plan_any_rows(16384, 7176, 2, false, false).vec &&
+            !plan_any_rows(513, 4095, 4, false, false).vec &&
+            plan_any_rows(512, 4095, 4, false, false).vec &&
+            plan_any_rows(16384, 14001, 2, true, false).vec &&
+            plan_any_rows(16384, 14001, 2, false, true).vec,
         "any-row forward without a residual");
   // Backward rows of any length: 2-byte ones of one wave of chunks go element by element, those
   // past 256 elements on short tensors only.
@@ -509,7 +512,7 @@ int main() {
     for (int eb = 2; eb <= 4; eb += 2) {
       const int V = 16 / eb, P = V / 2;
       for (int form = 0; form < 4; ++form) {
-        const RowPlan p = plan_any_rows(dim, eb, form & 1, form & 2);
+        const RowPlan p = plan_any_rows(16384, dim, eb, form & 1, form & 2);
         const bool wide_one_stream = form == 0 && dim / V > kAnyOneStreamChunks;
         CHECK(p.vec == (dim >= V && dim / V <= 2048 && !wide_one_stream), "any rows at %lld x %d",
               (long long)dim, eb);

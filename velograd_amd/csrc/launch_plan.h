@@ -137,16 +137,21 @@ constexpr int kAnyTwoChunks = 256;
 // generic kernel, whose 256-thread workgroups leave a CU more rows to overlap than one row group of
 // eight to sixteen waves.  Measured (8192 rows; generic kernel / any-row form, us): bf16 4099 32.0 /
 // 27.3, 6149 41.9 / 39.9, 7001 46.0 / 45.8, 7503 48.3 / 50.4, 8191 50.2 / 53.0, 10003 63.3 / 70.5,
-// 14001 89.1 / 100.7; fp32 3501 41.0 / 41.1, 4095 47.5 / 48.3, 5001 57.7 / 61.5, 8191 95.1 / 98.2.
+// 14001 89.1 / 100.7; fp32 3501 41.0 / 41.1, 4095 47.5 / 48.3, 5001 57.7 / 61.5, 8191 95.1 / 98.2.  A
+// few rows, which leave CUs idle either way, wait for one pass instead of two: 256 rows bf16 8191 5.5
+// / 4.7, 14001 8.5 / 6.1; 512 rows 6.5 / 6.0, 9.6 / 9.4; 768 rows 7.6 / 7.9, 11.5 / 13.5; fp32 8191 at
+// 512 rows 9.4 / 8.5, 768 11.7 / 13.0.
 constexpr int kAnyOneStreamChunks = 896;
+constexpr int64_t kAnyOneStreamRows = 512;
 // `residual`: the forward adds one; `quantised`: y is stored as fp8 or MX codes.
-inline RowPlan plan_any_rows(int64_t dim, int elem_bytes, bool residual, bool quantised) {
+inline RowPlan plan_any_rows(int64_t rows, int64_t dim, int elem_bytes, bool residual,
+                             bool quantised) {
   RowPlan p{false, 0, kGenericBlock, 1, kGenericBlock};
   if (elem_bytes != 2 && elem_bytes != 4) return p;
   const int V = 16 / elem_bytes;
   if (dim < V) return p;
   const int64_t chunks = dim / V;
-  if (!residual && !quantised && chunks > kAnyOneStreamChunks) return p;
+  if (!residual && !quantised && chunks > kAnyOneStreamChunks && rows > kAnyOneStreamRows) return p;
   const bool two = chunks > kWave && (!residual || quantised || chunks <= kAnyTwoChunks);
   const int nv = two || chunks > max_block_for_nv(1) ? 2 : 1;
   const int64_t tpr = (chunks + (int64_t)kWave * nv - 1) / ((int64_t)kWave * nv) * kWave;

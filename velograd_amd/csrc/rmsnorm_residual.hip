@@ -3125,7 +3125,8 @@ int32_t run_fwd(const char* what, int out, const void* x, const void* residual,
     elem_m = vg_plan::elem_per_lane(dim);
     if (elem_m > 0) p = vg_plan::plan_elem_rows(dim);
   } else if (!p.vec && out != kOutRopeI && aligned_elem) {
-    const RowPlan pa = vg_plan::plan_any_rows(dim, eb, residual != nullptr, out != kOutDtype);
+    const RowPlan pa =
+        vg_plan::plan_any_rows(rows, dim, eb, residual != nullptr, out != kOutDtype);
     if (pa.vec) {
       p = pa;
       any = true;
